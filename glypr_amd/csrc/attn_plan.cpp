@@ -6,36 +6,85 @@
 
 namespace glypr {
 
-// Queries per block: 16 AQS.  HD 512 runs one row of 16 queries (its two
-// 32 KB tile slots and 192 accumulator registers per lane leave no room for
-// more waves).  HD 256 takes 64-query blocks for long sequences and for many
-// rows (a batch of sequences): from 4096 rows the 64-query blocks' four-fold
-// K/V reuse beats the 16-query blocks' extra workgroups (32 x 512 rows:
-// 64 against 116 us per layer; 16 x 512: 44 against 62 us), below it the
-// 16-query blocks are as fast or faster (4 x 512: 24 against 30 us).
-int attn_qs(int64_t T, int64_t rows, int64_t hd) {
-  if (hd == 512) return 1;
-  return T > ATTN_SMALL_T || rows >= ATTN_QS4_ROWS ? 4 : 1;
-}
+namespace {
 
-// Tseg: the longest sequence (its key range sets the tile count); rows: the
-// padded rows of all sequences (they set the query blocks).
-int attn_kb_per_part(int64_t Tseg, int64_t rows, int64_t hd, int64_t nq, int64_t nkv,
-                     int64_t window, int* kparts) {
-  const int64_t aqb = 16 * attn_qs(Tseg, rows, hd);
-  const int64_t nqb = rows / aqb;
+// The most key tiles a block of `queries` query rows meets.
+int64_t key_tiles(int64_t Tseg, int64_t window, int64_t queries) {
   int64_t nkb = (Tseg + ATTN_AK - 1) / ATTN_AK;
   if (window > 0 && Tseg > window) {
-    int64_t band = (2 * window + aqb + ATTN_AK - 1) / ATTN_AK + 1;
+    const int64_t band = (2 * window + queries + ATTN_AK - 1) / ATTN_AK + 1;
     if (band < nkb) nkb = band;
   }
-  int64_t want = (ATTN_BLOCKS + nqb * nkv - 1) / (nqb * nkv);
-  if (want > (nkb + 1) / 2) want = (nkb + 1) / 2;
-  if (want < (nkb + 63) / 64) want = (nkb + 63) / 64;
-  if (want < 1) want = 1;
-  const int64_t per = (nkb + want - 1) / want;
-  *kparts = (int)((nkb + per - 1) / per);
-  return (int)per;
+  return nkb;
+}
+
+// Sets the cheapest of 1 .. most partitions over nkb key tiles for `blocks`
+// workgroups per partition and returns its cost in microseconds: every round
+// of 256 workgroups (one per CU: the K/V ring or the accumulators leave room
+// for one) takes `start` (launch, Q, first tile, epilogue) plus `tile` per key
+// tile, and a split pays for the f32 partials (written, then read by the
+// combine, ~5.5 TB/s) and the combine launch.  A grid that fills a round by
+// itself is never split.
+// `tile_full` takes the place of `tile` past 60 % of the CUs (clocks under load).
+double plan_parts(AttnPlan& p, int64_t blocks, int64_t nkb, double start, double tile,
+                  double tile_full, int64_t part_bytes) {
+  double best = 0;
+  int64_t most = nkb < ATTN_MAX_PARTS ? nkb : ATTN_MAX_PARTS;
+  if (blocks >= ATTN_BLOCKS) most = 1;
+  for (int64_t want = 1; want <= most; want++) {
+    const int64_t per = (nkb + want - 1) / want;
+    if ((nkb + per - 1) / per != want) continue;
+    const int64_t rounds = (blocks * want + ATTN_BLOCKS - 1) / ATTN_BLOCKS;
+    const bool full = blocks * want * 5 > ATTN_BLOCKS * 3;
+    const double c = rounds * (start + per * (full ? tile_full : tile)) +
+                     (want > 1 ? 3.0 + want * part_bytes * 2 / 5.5e6 : 0.0);
+    if (want == 1 || c < best) {
+      best = c;
+      p.per = (int)per;
+      p.kparts = (int)want;
+    }
+  }
+  return best;
+}
+
+}  // namespace
+
+// The choices with their measured starts and tile times (us):
+//   16-query blocks, 3 + 1.3 (head_dim 256) and 6.7 + 3.2 (512): few keys;
+//   64-query blocks (256), 13 + 0.52 per q head of the group: where they fill
+//     just one round and the 32 x 32 tiles leave SIMDs idle (32 sequences x 512
+//     rows of 3 heads: 41.7 against 55 us; T = 8192 of 3 heads: 249 against
+//     271 us);
+//   32 x 32 tiles, 5 + 0.8 (0.97 under load) and 11.5 + 2.05: everything longer (T = 1777,
+//     window 512: 49.9 -> 37.0 us with the prologue; T = 4000 of 3 heads: 118 ->
+//     87; T = 4000 of 4 heads, head_dim 512: 375 -> 185; T = 8192: 1472 -> 565).
+AttnPlan attn_plan(int64_t Tseg, int64_t rows, int64_t hd, int64_t nq, int64_t nkv,
+                   int64_t window, bool segments) {
+  const int64_t G = nq / nkv, part_bytes = rows * nq * hd * 4;
+  AttnPlan best{};
+  double best_cost = 0;
+  auto offer = [&](int waves, int qs, int64_t queries, int64_t blocks, double start,
+                   double tile, double tile_full) {
+    AttnPlan p{waves, qs, 0, 0};
+    const double c = plan_parts(p, nkv * blocks, key_tiles(Tseg, window, queries), start, tile,
+                                tile_full, part_bytes);
+    if (best.kparts == 0 || c < best_cost) {
+      best = p;
+      best_cost = c;
+    }
+  };
+  const bool wide = hd == 512;
+  offer(0, 1, 16, rows / 16, wide ? 6.7 : 3.0, wide ? 3.2 : 1.3,
+        wide ? 3.2 : 1.3);
+  if (!wide) offer(0, 4, 64, rows / 64, 13.0, 0.52 * G, 0.52 * G);
+  // Four column groups (32 queries of one head) per workgroup fill its CU's
+  // SIMDs.  With several sequences a workgroup stays within one, so within 64
+  // rows: two groups of one head, three of three heads.
+  const int waves = !segments || G % 2 == 0 ? 4 : G == 1 ? 2 : 3;
+  const int64_t queries = waves % G == 0 ? 32 * (waves / G) : 64;
+  offer(waves, 0, queries, ((rows >> 5) * G + waves - 1) / waves, wide ? 11.5 : 5.0,
+        wide ? 2.05 : 0.8, wide ? 2.05 : 0.97);
+  return best;
 }
 
 bool attention_rows_ok(int64_t rows, int64_t hd) {
@@ -47,36 +96,34 @@ bool attention_supported(int64_t T, int64_t nq, int64_t nkv, int64_t hd, int64_t
     return false;
   if (T <= 0) return true;
   if (!attention_rows_ok(T, hd)) return false;
-  int kparts;
-  attn_kb_per_part(T, attn_padded_len(T), hd, nq, nkv, window, &kparts);
-  return kparts <= 64;   // the combine holds one partition per lane
+  // the combine holds one partition per lane
+  return attn_plan(T, attn_padded_len(T), hd, nq, nkv, window, false).kparts <= 64;
 }
 
 size_t attention_scratch_floats(int64_t T, int64_t nq, int64_t nkv, int64_t hd, int64_t window,
                                 int64_t rows) {
   const int64_t tp = rows > 0 ? rows : attn_padded_len(T);
-  int kp;
-  attn_kb_per_part(T, tp, hd, nq, nkv, window, &kp);
+  int kp = 1;
+  for (const bool segments : {false, true}) {
+    const int k = attn_plan(T, tp, hd, nq, nkv, window, segments).kparts;
+    kp = k > kp ? k : kp;
+  }
   return (size_t)(kp * tp * nq * (hd + 2));
 }
 
 size_t attention_scratch_bound(int64_t max_t, int64_t cap_rows, int64_t nq, int64_t nkv,
                                int64_t hd, int64_t window) {
-  // For one tk, kparts depends on rows only through the query blocks:
-  // their count (want) and their size (16 or 64 queries, switching at
-  // ATTN_QS4_ROWS).  Every row count is visited until neither can change
-  // kparts any more: the blocks are 64 queries and they fill a round by
-  // themselves (nqb nkv >= ATTN_BLOCKS, so want = 1 and kparts = the clamp
-  // of the key tiles alone).  From there kparts is constant and the
-  // product kparts * rows peaks at the capacity.
+  // For one tk, the plan depends on rows only through the block counts and the
+  // partials' bytes.  Every row count is visited until the coarsest blocks (128
+  // queries: four groups of one head) fill a round by themselves: from there no choice
+  // splits, and kparts * rows = rows peaks at the capacity.
   size_t best = 0;
   for (int64_t tk = 32;; tk += 32) {
     if (tk > max_t) tk = max_t;
     for (int64_t rows = attn_padded_len(tk); rows <= cap_rows; rows += 64) {
       size_t sc = attention_scratch_floats(tk, nq, nkv, hd, window, rows);
       best = sc > best ? sc : best;
-      const int64_t aqb = 16 * attn_qs(tk, rows, hd);
-      if (rows >= ATTN_QS4_ROWS && (rows / aqb) * nkv >= ATTN_BLOCKS && rows < cap_rows) {
+      if (rows / 128 * nkv >= ATTN_BLOCKS && rows < cap_rows) {
         sc = attention_scratch_floats(tk, nq, nkv, hd, window, cap_rows);
         best = sc > best ? sc : best;
         break;

@@ -175,25 +175,20 @@ hipError_t launch_geglu_quant(const float* g, const float* u, int64_t u_stride, 
 // ---- k_attn.hip, attn_plan.cpp ----
 // Attention operands are padded to Tp = attn_padded_len(T) tokens.
 constexpr int64_t ATTN_TP_ALIGN = 64;
-// The partitioned kernels: keys per K/V tile; sequences up to ATTN_SMALL_T
-// use 16-query blocks (more blocks to spread), longer ones 64-query blocks
-// (each K/V tile serves 4x the queries; head_dim 256).
+// The partitioned kernels: keys per K/V tile, workgroups per round (one per
+// CU), and the most key partitions (the combine holds one per lane).
 constexpr int ATTN_AK = 32;
-constexpr int64_t ATTN_SMALL_T = 1024;
-// Key partitions: enough (query block, partition) items for one round of
-// workgroups (256 CUs), at most half the key tiles per partition and at most
-// 64 partitions (the combine holds one partition per lane).
 constexpr int64_t ATTN_BLOCKS = 256;
-// From this many padded rows (a batch of sequences) head_dim 256 takes
-// 64-query blocks.
-constexpr int64_t ATTN_QS4_ROWS = 4096;
-// Queries per block / 16 for the longest sequence T over `rows` padded rows.
-int attn_qs(int64_t T, int64_t rows, int64_t hd);
-// Key tiles per partition (returned) and the partition count (*kparts) for
-// the longest sequence Tseg (its key range sets the tile count) over `rows`
-// padded rows (they set the query blocks).
-int attn_kb_per_part(int64_t Tseg, int64_t rows, int64_t hd, int64_t nq, int64_t nkv,
-                     int64_t window, int* kparts);
+constexpr int64_t ATTN_MAX_PARTS = 64;
+// How the partitioned kernels run sequences of up to Tseg keys over `rows`
+// padded rows: the 32 x 32 tile kernel on workgroups of `waves` waves (qs 0),
+// or attn_partial_kernel in blocks of 16 qs queries; `kparts` partitions of
+// `per` key tiles.
+struct AttnPlan {
+  int waves, qs, per, kparts;
+};
+AttnPlan attn_plan(int64_t Tseg, int64_t rows, int64_t hd, int64_t nq, int64_t nkv,
+                   int64_t window, bool segments);
 inline int64_t attn_padded_len(int64_t t) { return (t + ATTN_TP_ALIGN - 1) / ATTN_TP_ALIGN * ATTN_TP_ALIGN; }
 // q16 [nq][Tp][hd], k16 [nkv][Tp][hd], vt16 [nkv][hd][Tp] (f16).  hd == 256.
 // seg (nullable, device int32 pairs [Tp][2]): row t holds position t - seg[t][0]
@@ -213,6 +208,14 @@ size_t attention_scratch_floats(int64_t T, int64_t nq, int64_t nkv, int64_t hd, 
 // attn_padded_len of it up to cap_rows (a multiple of 64).
 size_t attention_scratch_bound(int64_t max_t, int64_t cap_rows, int64_t nq, int64_t nkv,
                                int64_t hd, int64_t window);
+// The partitioned attention on 32 x 32 MFMA tiles (k_attn32.hip), for a plan
+// with qs 0; with one partition it writes the context itself, otherwise
+// part_o / part_ml as attn_partial_kernel does.
+hipError_t launch_attn_tile32(const uint16_t* q16, const uint16_t* k16, const uint16_t* vt16,
+                              float* part_o, float* part_ml, int64_t T, int64_t Tp, int64_t nq,
+                              int64_t nkv, int64_t hd, int64_t window, const AttnPlan& plan,
+                              const int32_t* seg, float* ctx, int8_t* cq, float* dc, uint16_t* cb,
+                              hipStream_t s);
 // Whether launch_attention runs this geometry: head_dim 256 or 512, nq / nkv
 // in 1..4, at most 64 key partitions at T and attention_rows_ok (T <= 0: any
 // length).

@@ -17,6 +17,7 @@
 // normalisation are f32.  The K and V roundings dominate: carrying Q and P in
 // two f16 parts as well would cut the context error by only ~20 % at twice the
 // MFMA work.
+#include "attn_common.hpp"
 #include "device_common.hpp"
 #include "internal.hpp"
 
@@ -246,37 +247,9 @@ hipError_t launch_qkv_post(const float* qkv, int64_t T, int64_t Tp, int64_t nq, 
 // B (32 x 16): column l%16, same k; D (16 x 16): column l%16, rows 4(l/16)+r.
 // ---------------------------------------------------------------------------
 constexpr int AK = ATTN_AK;       // keys per tile
-constexpr float ATTN_TAU = 8.0f;  // lazy-rescale threshold (natural log): p <= e^8 ~ 2981
-constexpr float ATTN_LOG2E = 1.44269504f;
 static_assert(ATTN_TP_ALIGN % 64 == 0, "query blocks (16 or 64) must tile the padded length");
 
 typedef float v4f_ __attribute__((ext_vector_type(4)));
-
-// Lane pairs (l, l ^ 16) and (l, l ^ 32) through gfx950's permlane swaps:
-// v_permlane16_swap / v_permlane32_swap of a value with itself return, in
-// every lane, the lane's own value and its partner's (in either order), all
-// in VALU — no LDS round trip as with ds_bpermute.  max and + over the pair
-// are order-independent, so each equals op(v, v[l ^ 16]) (resp. l ^ 32).
-__device__ __forceinline__ float pair_max16(float v) {
-  const auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false,
-                                                  false);
-  return fmaxf(__uint_as_float(p[0]), __uint_as_float(p[1]));
-}
-__device__ __forceinline__ float pair_max32(float v) {
-  const auto p = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false,
-                                                  false);
-  return fmaxf(__uint_as_float(p[0]), __uint_as_float(p[1]));
-}
-__device__ __forceinline__ float pair_sum16(float v) {
-  const auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false,
-                                                  false);
-  return __uint_as_float(p[0]) + __uint_as_float(p[1]);
-}
-__device__ __forceinline__ float pair_sum32(float v) {
-  const auto p = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false,
-                                                  false);
-  return __uint_as_float(p[0]) + __uint_as_float(p[1]);
-}
 
 // LDS swizzles (16-byte chunk c of row r is stored at chunk c ^ swz(r)),
 // chosen by measurement: with them the fragment reads show no
@@ -1008,7 +981,9 @@ static hipError_t run_attention(const f16* q, const f16* k, const f16* v, float*
                                 int64_t nq, int64_t nkv, int64_t window, hipStream_t s,
                                 uint16_t* cb, const int2* seg, int64_t seg_max) {
   const int64_t G = nq / nkv;
-  if (HD == 256 && !seg && Tp <= ATTN_SHORT_TP && G <= 3) {
+  // (two kv heads double its grid: past 1280 rows of both it takes three rounds
+  // and more, where the tiles win: T = 850, 37.7 against 30.3 us)
+  if (HD == 256 && !seg && Tp <= ATTN_SHORT_TP && nkv * Tp <= 1280 && G <= 3) {
     // one short sequence: the single-launch slice kernel
     const int64_t items = nkv * (Tp / 16) * (HD / ASH_DS);
     const unsigned grid = (unsigned)((items + 7) / 8 * 8);
@@ -1021,32 +996,39 @@ static hipError_t run_attention(const f16* q, const f16* k, const f16* v, float*
     return hipGetLastError();
   }
   const int64_t Tk = seg ? seg_max : T;   // the longest key range
-  const int aqs = attn_qs(Tk, Tp, HD);
-  int kparts;
-  const int per = attn_kb_per_part(Tk, Tp, HD, nq, nkv, window, &kparts);
-  if (kparts > 64) return hipErrorInvalidValue;   // the combine holds one partition per lane
+  const AttnPlan plan = attn_plan(Tk, Tp, HD, nq, nkv, window, seg != nullptr);
+  const int aqs = plan.qs, per = plan.per, kparts = plan.kparts;
   float* part_o = scratch;
   float* part_ml = scratch + (int64_t)kparts * Tp * nq * HD;
-  const int64_t items = nkv * kparts * (Tp / (16 * aqs));
-  const unsigned grid = (unsigned)((items + 7) / 8 * 8);
-#define GLYPR_ATTN_CASE(GG, QS)                                                                  \
-  if (G == GG && aqs == QS)                                                                      \
-    attn_partial_kernel<HD, GG, QS><<<grid, GG * QS * 64, 0, s>>>(                               \
-        q, k, v, part_o, part_ml, (int)T, (int)Tp, (int)nq, (int)nkv, (int)window, per, kparts, \
-        seg, ctx, cq, dc, cb);
-  if constexpr (HD == 256) {
-    GLYPR_ATTN_CASE(1, 1) else GLYPR_ATTN_CASE(1, 4)
-    else GLYPR_ATTN_CASE(2, 1) else GLYPR_ATTN_CASE(2, 4)
-    else GLYPR_ATTN_CASE(3, 1) else GLYPR_ATTN_CASE(3, 4)
-    else GLYPR_ATTN_CASE(4, 1) else GLYPR_ATTN_CASE(4, 4)
-    else return hipErrorInvalidValue;
+  hipError_t e;
+  if (plan.qs == 0) {
+    e = launch_attn_tile32(reinterpret_cast<const uint16_t*>(q),
+                           reinterpret_cast<const uint16_t*>(k),
+                           reinterpret_cast<const uint16_t*>(v), part_o, part_ml, T, Tp, nq, nkv,
+                           HD, window, plan, reinterpret_cast<const int32_t*>(seg), ctx, cq, dc,
+                           cb, s);
   } else {
-    GLYPR_ATTN_CASE(1, 1) else GLYPR_ATTN_CASE(2, 1)
-    else GLYPR_ATTN_CASE(3, 1) else GLYPR_ATTN_CASE(4, 1)
-    else return hipErrorInvalidValue;
-  }
+    const int64_t items = nkv * kparts * (Tp / (16 * aqs));
+    const unsigned grid = (unsigned)((items + 7) / 8 * 8);
+#define GLYPR_ATTN_CASE(GG, QS)                                                                  \
+    if (G == GG && aqs == QS)                                                                      \
+      attn_partial_kernel<HD, GG, QS><<<grid, GG * QS * 64, 0, s>>>(                               \
+          q, k, v, part_o, part_ml, (int)T, (int)Tp, (int)nq, (int)nkv, (int)window, per, kparts, \
+          seg, ctx, cq, dc, cb);
+    if constexpr (HD == 256) {
+      GLYPR_ATTN_CASE(1, 1) else GLYPR_ATTN_CASE(1, 4)
+      else GLYPR_ATTN_CASE(2, 1) else GLYPR_ATTN_CASE(2, 4)
+      else GLYPR_ATTN_CASE(3, 1) else GLYPR_ATTN_CASE(3, 4)
+      else GLYPR_ATTN_CASE(4, 1) else GLYPR_ATTN_CASE(4, 4)
+      else return hipErrorInvalidValue;
+    } else {
+      GLYPR_ATTN_CASE(1, 1) else GLYPR_ATTN_CASE(2, 1)
+      else GLYPR_ATTN_CASE(3, 1) else GLYPR_ATTN_CASE(4, 1)
+      else return hipErrorInvalidValue;
+    }
 #undef GLYPR_ATTN_CASE
-  hipError_t e = hipGetLastError();
+    e = hipGetLastError();
+  }
   if (e != hipSuccess || kparts == 1) return e;   // one partition: the partial wrote ctx
   attn_combine_kernel<HD><<<(unsigned)((T * nq + 3) / 4), 256, 0, s>>>(
       part_o, part_ml, (int)T, (int)Tp, (int)nq, kparts, ctx, cq, dc, cb);
