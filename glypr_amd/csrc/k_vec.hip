@@ -17,7 +17,8 @@
 //    i32 sums, so it runs on v_mfma_i32_16x16x64_i8: a wave holds 16 database
 //    rows against up to 64 queries, streaming K in 64-byte steps (16 bytes per
 //    lane); the database is read once per 64-query group, and for the cosine
-//    its row norms are summed from the same fragments.  Integer sums are
+//    its row norms are summed from the same fragments (v_dot4).  Rows of the MRL
+//    dims keep the queries in LDS.  Integer sums are
 //    order-free, so the result equals the reference's 4-lane sum bit for bit.
 #include "device_common.hpp"
 #include "internal.hpp"
@@ -175,14 +176,100 @@ __device__ __forceinline__ v4i load16(const int8_t* base, int64_t row, int64_t d
   return v;
 }
 
-__device__ __forceinline__ int32_t sq_sum16(v4i v) {
-  int32_t s = 0;
+// + the sum of the squares of 16 bytes (four v_dot4_i32_i8; exact in i32)
+__device__ __forceinline__ int32_t sq_sum16(v4i v, int32_t s) {
 #pragma unroll
-  for (int e = 0; e < 16; e++) {
-    const int32_t b = (int8_t)(v[e >> 2] >> (8 * (e & 3)));
-    s += b * b;
-  }
+  for (int e = 0; e < 4; e++) s = __builtin_amdgcn_sdot4(v[e], v[e], s, false);
   return s;
+}
+
+// int8_cosine_similarity's last step from the product and both squared norms'
+// roots (0 stands for a zero norm: the root of a positive integer is >= 1).
+__device__ __forceinline__ float cosine_of(int32_t dot, float ra, float rb) {
+  const float c = fminf(fmaxf((float)dot / (ra * rb), -1.0f), 1.0f);
+  return (ra != 0.0f && rb != 0.0f) ? c : 0.0f;
+}
+
+// All-pairs int8 products for rows of KS x 64 bytes: int8_pairs_kernel's tiles
+// (16 database rows x MT tiles of 16 queries per wave), with the queries kept
+// in LDS as MFMA fragments ([tile][step][lane][16 B]: conflict-free 1 KB reads)
+// for all the tiles a workgroup walks, and a database tile's KS loads all in
+// flight before its first product.  The cosine's query norms are summed here
+// too, from the fragments, so the call is one launch.
+// Bound: the database's bytes.  24 queries x 200,003 rows x 768: 60.0 us (norms
+// by 32 shifts and multiplies per 16 bytes, queries re-read per tile) plus a
+// 5 us norm launch -> 35 us (the call with its encode 64.5 -> 39.8); 64 x 90,000:
+// 56.2 -> 24.1 us, 1 x 200,003: 41.1 -> 30.2 us (5.1 TB/s, the card's copy rate).
+template <int MT, int KS, bool COS>
+__global__ void __launch_bounds__(256, 2) int8_pairs_lds_kernel(
+    const int8_t* __restrict__ a, int na, const int8_t* __restrict__ b, int64_t nb,
+    int32_t* __restrict__ out_d, float* __restrict__ out_c) {
+  constexpr int DIM = 64 * KS;
+  __shared__ v4i qa[MT * KS * 64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int l16 = lane & 15, lq = lane >> 4;
+  const int i0 = (int)blockIdx.y * 16 * MT;
+  for (int f = wave; f < MT * KS; f += 4) {   // fragment f = tile f / KS, step f % KS
+    const int i = i0 + 16 * (f / KS) + l16;
+    qa[f * 64 + lane] = *reinterpret_cast<const v4i*>(
+        a + (int64_t)(i < na ? i : na - 1) * DIM + 64 * (f % KS) + 16 * lq);
+  }
+  __syncthreads();
+  float ra[MT][4];   // roots of the norms of queries 16 t + 4 lq + r
+  if constexpr (COS) {
+#pragma unroll
+    for (int t = 0; t < MT; t++) {
+      int32_t n = 0;
+#pragma unroll
+      for (int k = 0; k < KS; k++) n = sq_sum16(qa[(t * KS + k) * 64 + lane], n);
+      n += __shfl_xor(n, 16);
+      n += __shfl_xor(n, 32);
+      const float root = sqrtf((float)n);   // query 16 t + l16
+#pragma unroll
+      for (int r = 0; r < 4; r++) ra[t][r] = __shfl(root, 4 * lq + r);
+    }
+  }
+  const int64_t step = (int64_t)gridDim.x * 64;
+  for (int64_t j0 = ((int64_t)blockIdx.x * 4 + wave) * 16; j0 < nb; j0 += step) {
+    const int64_t j = j0 + l16;
+    const int8_t* row = b + (j < nb ? j : nb - 1) * DIM + 16 * lq;
+    v4i bf[KS];
+#pragma unroll
+    for (int k = 0; k < KS; k++) bf[k] = *reinterpret_cast<const v4i*>(row + 64 * k);
+    v4i acc[MT];
+#pragma unroll
+    for (int t = 0; t < MT; t++) acc[t] = v4i{0, 0, 0, 0};
+    int32_t nsq = 0;
+    // the query fragments are read again for every tile (the opaque index
+    // keeps them out of MT x KS x 4 registers, which would cost the waves)
+    int at = lane;
+    asm volatile("" : "+v"(at));
+#pragma unroll
+    for (int k = 0; k < KS; k++) {
+      if (COS) nsq = sq_sum16(bf[k], nsq);
+#pragma unroll
+      for (int t = 0; t < MT; t++)
+        acc[t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(qa[(t * KS + k) * 64 + at], bf[k],
+                                                       acc[t], 0, 0, 0);
+    }
+    float rb = 0.0f;
+    if (COS) {
+      nsq += __shfl_xor(nsq, 16);
+      nsq += __shfl_xor(nsq, 32);
+      rb = sqrtf((float)nsq);
+    }
+    if (j < nb) {
+#pragma unroll
+      for (int t = 0; t < MT; t++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          const int i = i0 + 16 * t + 4 * lq + r;
+          if (i >= na) continue;
+          if (COS) out_c[(int64_t)i * nb + j] = cosine_of(acc[t][r], ra[t][r], rb);
+          else out_d[(int64_t)i * nb + j] = acc[t][r];
+        }
+    }
+  }
 }
 
 // All-pairs int8 dot on MFMA.  A wave: database rows j0 .. j0+15 (output
@@ -213,7 +300,7 @@ __global__ void __launch_bounds__(256) int8_pairs_kernel(
   for (int64_t k0 = 0; k0 < dim; k0 += 64) {
     const int64_t k = k0 + 16 * lq;
     const v4i bf = load16<FAST>(b, jr, dim, k);
-    if (COS) nsq += sq_sum16(bf);
+    if (COS) nsq = sq_sum16(bf, nsq);
 #pragma unroll
     for (int t = 0; t < MT; t++) {
       const v4i af = load16<FAST>(a, ir[t], dim, k);
@@ -236,12 +323,7 @@ __global__ void __launch_bounds__(256) int8_pairs_kernel(
         out_d[i * nb + j] = acc[t][r];
       } else {
         const int32_t nai = norm_a[i];
-        float c = 0.0f;
-        if (nai != 0 && nsq != 0) {
-          const float denom = sqrtf((float)nai) * sqrtf((float)nsq);
-          c = fminf(fmaxf((float)acc[t][r] / denom, -1.0f), 1.0f);
-        }
-        out_c[i * nb + j] = c;
+        out_c[i * nb + j] = cosine_of(acc[t][r], sqrtf((float)nai), sqrtf((float)nsq));
       }
     }
 }
@@ -281,6 +363,46 @@ hipError_t run_int8_pairs_mt(const int8_t* a, int64_t na, const int8_t* b, int64
     int8_pairs_kernel<MT, false, COS><<<grid, 256, 0, s>>>(a, na, b, nb, dim, out_d, norm_a,
                                                            out_c);
   return hipGetLastError();
+}
+
+// Two workgroups per CU (2, 3 and 4 measured 39.8, 41.9 and 44.5 us at 24 queries
+// x 200,003 rows x 768).
+constexpr int64_t PAIRS_WG = 512;
+
+// The LDS kernel for rows of 64, 128, 256, 512, 768 or 1024 bytes (the MRL
+// dims); up to 8 workgroups per CU, each walking the tiles that are left.
+template <int MT, bool COS>
+bool run_int8_pairs_lds(const int8_t* a, int64_t na, const int8_t* b, int64_t nb, int64_t dim,
+                        int32_t* out_d, float* out_c, hipStream_t s) {
+  if (na > (int64_t(1) << 24)) return false;
+  // whole rounds of workgroups that fit at once, each walking as many tiles
+  const int64_t tiles = (nb + 63) / 64, walk = (tiles + PAIRS_WG - 1) / PAIRS_WG;
+  const dim3 grid((unsigned)((tiles + walk - 1) / walk),
+                  (unsigned)((na + 16 * MT - 1) / (16 * MT)));
+  if (grid.y > 65535) return false;
+#define PAIRS_CASE(K)                                                                           \
+  case 64 * K:                                                                                  \
+    int8_pairs_lds_kernel<MT, K, COS><<<grid, 256, 0, s>>>(a, (int)na, b, nb, out_d, out_c);   \
+    return true;
+  switch (dim) {
+    PAIRS_CASE(1)
+    PAIRS_CASE(2)
+    PAIRS_CASE(4)
+    PAIRS_CASE(8)
+    PAIRS_CASE(12)
+    PAIRS_CASE(16)
+    default: return false;
+  }
+#undef PAIRS_CASE
+}
+
+// Whether the LDS kernel took the call.
+template <bool COS>
+bool int8_pairs_lds(const int8_t* a, int64_t na, const int8_t* b, int64_t nb, int64_t dim,
+                    int32_t* out_d, float* out_c, hipStream_t s) {
+  if (na <= 16) return run_int8_pairs_lds<1, COS>(a, na, b, nb, dim, out_d, out_c, s);
+  if (na <= 32) return run_int8_pairs_lds<2, COS>(a, na, b, nb, dim, out_d, out_c, s);
+  return run_int8_pairs_lds<4, COS>(a, na, b, nb, dim, out_d, out_c, s);
 }
 
 // Query tiles per wave: just enough 16-row tiles for na (at most 4 per pass).
@@ -335,12 +457,14 @@ hipError_t launch_binary_cosine(const uint64_t* a, int64_t na, const uint64_t* b
 hipError_t launch_int8_dot(const int8_t* a, int64_t na, const int8_t* b, int64_t nb, int64_t dim,
                            int32_t* out, hipStream_t s) {
   if (na == 0 || nb == 0) return hipSuccess;
+  if (int8_pairs_lds<false>(a, na, b, nb, dim, out, nullptr, s)) return hipGetLastError();
   return run_int8_pairs<false>(a, na, b, nb, dim, out, nullptr, nullptr, s);
 }
 
 hipError_t launch_int8_cosine(const int8_t* a, int64_t na, const int8_t* b, int64_t nb,
                               int64_t dim, int32_t* norms, float* out, hipStream_t s) {
   if (na == 0 || nb == 0) return hipSuccess;
+  if (int8_pairs_lds<true>(a, na, b, nb, dim, nullptr, out, s)) return hipGetLastError();
   int8_row_norms_kernel<<<(unsigned)((na + 3) / 4), 256, 0, s>>>(a, na, dim, norms);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
