@@ -1042,22 +1042,24 @@ hipError_t run_pro(const float* x, const float* nw, float eps, const int8_t* wq,
 }
 
 // ---------------------------------------------------------------------------
-// Large-M variant (M > 2048: batched sequences, long contexts).  The exact
+// Large-M variant (M > 2048: batched sequences, long contexts; the plain GEMM
+// from about 1000 rows, see tiles_beat_small).  The exact
 // epilogue (3 VALU ops per output and block) binds.  On gfx950 the MFMA pipe
 // and the VALU do not overlap for this MFMA -> dependent-epilogue pattern, so
 // the cost per output and block is (VALU ops + MFMA cycles): the kernel uses
 // the full-rate v_mfma_i32_32x32x32_i8 (2 cycles per output and block, half
 // of the 16x16x32 form).  Structure:
-//  - 4 waves stacked along M; wave w owns rows 32w..32w+31 of a 128 x 128
-//    tile and all 128 columns (4 MFMA tiles of 32 x 32, 64 accumulators);
+//  - WMW waves along M by WNW along N, each 32 rows x TN MFMA tiles of 32
+//    columns: 4 x 1 x 4 (128 x 128 tiles, the GeGLU's), 2 x 2 x 1 (64 x 64) and
+//    2 x 2 x 2 (64 x 128), see big_tile;
 //  - every stage (128 bytes of K = 4 blocks) arrives by LDS DMA into a
-//    two-slot ring: A tile [128][128 B] and B tile [128][128 B] (16-byte
+//    two-slot ring: A tile [BM][128 B] and B tile [BN][128 B] (16-byte
 //    chunk c of row r at c ^ ((r >> 1) & 7): conflict-free ds_read_b128),
 //    then the A and B scales of the stage as [block][row] f32 (dword DMA), so
 //    the 16 row scales of a lane's 32 x 32 outputs are 4 ds_read_b128;
-//    48 units, 12 per wave: "stage s has landed" is vmcnt(0) + barrier and
-//    the next stage streams in under the current stage's compute;
-//  - 2 workgroups per CU (72 KB LDS, <= 256 VGPRs each);
+//    (128 x 128: 48 units, 12 per wave) "stage s has landed" is vmcnt(0) +
+//    barrier and the next stage streams in under the current stage's compute;
+//  - 2 workgroups per CU (72 or 54 KB LDS, <= 256 VGPRs each), 4 of 64 x 64;
 //  - the tile order is XCD-aware: the 8 XCDs get contiguous ranges of the
 //    row-major tile list, so the tiles sharing an A row block share an L2.
 // Rows past M/N are clamped to a valid row (their outputs are never stored).
@@ -1067,17 +1069,15 @@ hipError_t run_pro(const float* x, const float* nw, float eps, const int8_t* wq,
 // is a 32-lane reduction, and each wave derives its 64 (row, block) scales one
 // per lane through a per-wave LDS table instead of repeating the divisions.
 // ---------------------------------------------------------------------------
-constexpr int BIG_BM = 128, BIG_BN = 128;
-
 __device__ __forceinline__ int big_swz(int row) { return (row >> 1) & 7; }
 
-template <bool GEGLU, bool F2>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
+template <int WMW, int WNW, int TN, bool GEGLU, bool F2>
+__global__ void __launch_bounds__(WMW * WNW * 64) __attribute__((amdgpu_waves_per_eu(TN == 4 ? 2 : 4)))
 gemm_i8_big_kernel(const int8_t* __restrict__ A, const float* __restrict__ dA,
                    const int8_t* __restrict__ B, const float* __restrict__ dB,
                    float* __restrict__ C, int8_t* __restrict__ Hq, float* __restrict__ dH,
                    int M, int N, int K, int ldc, int F, int tiles_n) {
-  constexpr int NW = 4, TN = 4;
+  constexpr int NW = WMW * WNW, BIG_BM = 32 * WMW, BIG_BN = 32 * TN * WNW;
   constexpr int UA = BIG_BM / 8, UB = BIG_BN / 8;        // 1 KB operand units
   constexpr int USA = KB * BIG_BM / 64, USB = KB * BIG_BN / 64;   // 256 B scale units
   constexpr int NU = UA + UB + USA + USB;
@@ -1090,6 +1090,7 @@ gemm_i8_big_kernel(const int8_t* __restrict__ A, const float* __restrict__ dA,
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave % WMW, wn = wave / WMW;
   // XCD-aware tile id: workgroup i runs on XCD i % 8 (the grid is exactly
   // the tile count, taken from the arguments rather than gridDim)
   const int nblk = ((M + BIG_BM - 1) / BIG_BM) * tiles_n, id = blockIdx.x;
@@ -1153,18 +1154,18 @@ gemm_i8_big_kernel(const int8_t* __restrict__ A, const float* __restrict__ dA,
   issue(0, 0);
 
   const int lrow = lane & 31, lhalf = lane >> 5;
-  const int arow = wave * 32 + lrow;
+  const int arow = wm * 32 + lrow;
   // operand chunk of block kb: bytes 32 kb + 16 lhalf of the row
   int offA[KB], offB[KB];
 #pragma unroll
   for (int kb = 0; kb < KB; kb++) {
     const int ch = 2 * kb + lhalf;
     offA[kb] = arow * BK + ((ch ^ big_swz(arow)) << 4);
-    offB[kb] = (BIG_BM + lrow) * BK + ((ch ^ big_swz(lrow)) << 4);   // tile tn: + 32 tn rows
+    offB[kb] = (BIG_BM + wn * 32 * TN + lrow) * BK + ((ch ^ big_swz(lrow)) << 4);   // tile tn: + 32 tn rows
   }
   // A scales of rows 32 w + 8 g + 4 lhalf + (0..3): b128 g at + 32 g
-  const int offX = OFF_SA + (wave * 32 + 4 * lhalf) * 4;
-  const int offW = OFF_SB + lrow * 4;   // B scale of tile tn, block kb: + (kb * 128 + 32 tn) * 4
+  const int offX = OFF_SA + (wm * 32 + 4 * lhalf) * 4;
+  const int offW = OFF_SB + (wn * 32 * TN + lrow) * 4;   // B scale of tile tn, block kb: + (kb * 128 + 32 tn) * 4
   v16i magic;
 #pragma unroll
   for (int i = 0; i < 16; i++) magic[i] = MAGIC;
@@ -1205,11 +1206,11 @@ gemm_i8_big_kernel(const int8_t* __restrict__ A, const float* __restrict__ dA,
   }
 
   // output rows of register r: 32 w + 8 (r >> 2) + 4 lhalf + (r & 3)
-  const int row0 = m0 + wave * 32 + 4 * lhalf;
+  const int row0 = m0 + wm * 32 + 4 * lhalf;
   if constexpr (!GEGLU) {
 #pragma unroll
     for (int tn = 0; tn < TN; tn++) {
-      const int gn = n0 + 32 * tn + lrow;
+      const int gn = n0 + wn * 32 * TN + 32 * tn + lrow;
 #pragma unroll
       for (int r = 0; r < 16; r++) {
         const int gm = row0 + 8 * (r >> 2) + (r & 3);
@@ -1221,56 +1222,108 @@ gemm_i8_big_kernel(const int8_t* __restrict__ A, const float* __restrict__ dA,
     // value of geglu(acc[2p][r], acc[2p+1][r]).  Scale table per wave in the
     // ring slot of stage nst - 2, which every wave finished before the last
     // barrier: amax[lhalf][p][r], then (id, dq) per entry.
+    constexpr int TE = 16 * TN;   // table entries: (lhalf, p, r)
+    static_assert(TN % 2 == 0, "gate and up tiles in pairs");
     const int nbh = F / QK;
-    float* tab = reinterpret_cast<float*>(ring + (((nst - 1) & 1) ^ 1) * SLOT) + wave * 192;
-    float h[2][16];
+    float* tab = reinterpret_cast<float*>(ring + (((nst - 1) & 1) ^ 1) * SLOT) + wave * TE * 3;
+    float h[TN / 2][16];
 #pragma unroll
-    for (int p = 0; p < 2; p++)
+    for (int p = 0; p < TN / 2; p++)
 #pragma unroll
       for (int r = 0; r < 16; r++) {
         h[p][r] = geglu_scalar(acc[2 * p][r], acc[2 * p + 1][r]);
         const float v = max32_hi(fmaxf(0.0f, fabsf(h[p][r])));
-        if (lrow == 31) tab[lhalf * 32 + p * 16 + r] = v;
+        if (lrow == 31) tab[lhalf * (TE / 2) + p * 16 + r] = v;
       }
     // LDS serves a wave's accesses in order; the fences keep the compiler
     // from moving the table accesses across each other.
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    {
+    if (TE >= 64 || lane < TE) {
       const QScale q = q8_scale(tab[lane]);
-      tab[64 + lane] = q.id;
-      tab[128 + lane] = q.dq;
+      tab[TE + lane] = q.id;
+      tab[2 * TE + lane] = q.dq;
     }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    const int c = hc0;
+    const int c = hc0 + wn * 16 * TN;
 #pragma unroll
-    for (int p = 0; p < 2; p++) {
+    for (int p = 0; p < TN / 2; p++) {
       const int hb = c + 32 * p;   // first column of the h block
 #pragma unroll
       for (int r = 0; r < 16; r++) {
         const int gm = row0 + 8 * (r >> 2) + (r & 3);
-        const int e = lhalf * 32 + p * 16 + r;
+        const int e = lhalf * (TE / 2) + p * 16 + r;
         if (gm < M && hb < F) {
-          Hq[(int64_t)gm * F + hb + lrow] = (int8_t)quant_round(h[p][r] * tab[64 + e]);
-          if (lrow == 0) dH[(int64_t)gm * nbh + (hb >> 5)] = tab[128 + e];
+          Hq[(int64_t)gm * F + hb + lrow] = (int8_t)quant_round(h[p][r] * tab[TE + e]);
+          if (lrow == 0) dH[(int64_t)gm * nbh + (hb >> 5)] = tab[2 * TE + e];
         }
       }
     }
   }
 }
 
+template <int WMW, int WNW, int TN, bool GEGLU, bool F2>
+hipError_t run_big_tile(const int8_t* xq, const float* dx, const int8_t* wq, const float* dw,
+                        float* y, int8_t* hq, float* dh, int64_t M, int64_t Nrows, int64_t K,
+                        int64_t ldc, int64_t F, hipStream_t s) {
+  constexpr int BM = 32 * WMW, BN = 32 * TN * WNW;
+  const int64_t tiles_n = (Nrows + BN - 1) / BN;
+  const int64_t tiles = ((M + BM - 1) / BM) * tiles_n;
+  gemm_i8_big_kernel<WMW, WNW, TN, GEGLU, F2><<<dim3((unsigned)tiles), WMW * WNW * 64, 0, s>>>(
+      xq, dx, wq, dw, y, hq, dh, (int)M, (int)Nrows, (int)K, (int)ldc, (int)F, (int)tiles_n);
+  return hipGetLastError();
+}
+
+// The plain GEMM's tile: 0 = 128 x 128 (wave 32 x 128), 1 = 64 x 64 (32 x 32),
+// 2 = 64 x 128 (32 x 64).  A wave's column tile and K block (one MFMA and its
+// exact epilogue) costs 0.15-0.2 us alone on its SIMD and ~0.1-0.13 us of a
+// shared one, so what decides is how the grid's waves spread: the estimate below
+// (us, with the measured cost per tile-block for 1 .. 4 workgroups per CU)
+// deals the workgroups out over 256 CUs in rounds of what fits a CU.
+// Measured, 128 x 128 -> chosen: 2500 x 768 x 768 19.2 -> 10.0 us (64 x 64),
+// 3000 x 768 x 1280 16.8 -> 13.0 (64 x 128), 4800 x 2048 x 512 44 -> 26,
+// 12000 x 768 x 768 39.6 -> 29.5; 6000 x 768 x 1280 stays (22.9 against 25.5), as
+// do 16384 rows of 1280 or 2304 columns (61 against 63).
+inline double big_cost(int64_t M, int64_t N, int64_t K, int tile) {
+  static const double f0[] = {0.15, 0.20}, f1[] = {0.216, 0.29, 0.39, 0.53}, f2[] = {0.17, 0.22};
+  const int64_t bm = tile == 0 ? 128 : 64, bn = tile == 1 ? 64 : 128;
+  const int fit = tile == 1 ? 4 : 2, cols = tile == 0 ? 4 : tile == 1 ? 1 : 2;
+  const double* f = tile == 0 ? f0 : tile == 1 ? f1 : f2;
+  const int64_t n = (((M + bm - 1) / bm) * ((N + bn - 1) / bn) + 255) / 256;
+  const int64_t rounds = n / fit;
+  const int rest = (int)(n % fit);
+  const double blocks = (double)(K / QK) * cols;
+  return 3.0 + blocks * (rounds * f[fit - 1] + (rest ? f[rest - 1] : 0.0)) +
+         (tile == 1 ? 0.0 : (double)(rounds + (rest != 0) - 1));
+}
+inline int big_tile(int64_t M, int64_t N, int64_t K) {
+  const double c0 = big_cost(M, N, K, 0), c1 = big_cost(M, N, K, 1), c2 = big_cost(M, N, K, 2);
+  return c1 <= c0 && c1 <= c2 ? 1 : c2 < c0 ? 2 : 0;
+}
+// Whether up to 2048 rows the 64 x 64 tiles beat gemm_i8_small_kernel, whose
+// 16 x 32 tiles cost 2.7 us + 0.21 us per thousand 32 x 32 x 32 blocks (1213 x
+// 768 x 1280: 9.5 -> 8.3 us; 2048 x 512 x 3072: 22.2 -> 15.5; 1213 x 768 x 768
+// stays: 7.7 against 8.2).
+inline bool tiles_beat_small(int64_t M, int64_t N, int64_t K) {
+  const double work = (double)((M + 31) / 32) * ((N + 31) / 32) * (K / QK);
+  return big_cost(M, N, K, 1) < 2.7 + 0.00021 * work;
+}
+
 template <bool GEGLU, bool F2>
 hipError_t run_big(const int8_t* xq, const float* dx, const int8_t* wq, const float* dw,
                    float* y, int8_t* hq, float* dh, int64_t M, int64_t Nrows, int64_t K,
                    int64_t ldc, int64_t F, hipStream_t s) {
-  const int64_t tiles_n = (Nrows + BIG_BN - 1) / BIG_BN;
-  const int64_t tiles = ((M + BIG_BM - 1) / BIG_BM) * tiles_n;
-  gemm_i8_big_kernel<GEGLU, F2><<<dim3((unsigned)tiles), 256, 0, s>>>(
-      xq, dx, wq, dw, y, hq, dh, (int)M, (int)Nrows, (int)K, (int)ldc, (int)F, (int)tiles_n);
-  return hipGetLastError();
+  if constexpr (!GEGLU) {
+    const int tile = big_tile(M, Nrows, K);
+    if (tile == 1)
+      return run_big_tile<2, 2, 1, false, F2>(xq, dx, wq, dw, y, hq, dh, M, Nrows, K, ldc, F, s);
+    if (tile == 2)
+      return run_big_tile<2, 2, 2, false, F2>(xq, dx, wq, dw, y, hq, dh, M, Nrows, K, ldc, F, s);
+  }
+  return run_big_tile<4, 1, 4, GEGLU, F2>(xq, dx, wq, dw, y, hq, dh, M, Nrows, K, ldc, F, s);
 }
 
 // The large-M kernel addresses operands with 32-bit offsets.
@@ -1780,6 +1833,8 @@ hipError_t gemm_i8_routed(const int8_t* xq, const float* dx, const int8_t* wq, c
                           hipStream_t s) {
   switch (gemm_i8_route(M, N, K)) {
     case GEMM_ROUTE_SMALL:
+      if (big_ok(M, N, K) && tiles_beat_small(M, N, K))
+        return run_big<false, F2>(xq, dx, wq, dw, y, nullptr, nullptr, M, N, K, ldc, 0, s);
       return run_small<1, 2, 1, false, F2, 3>(xq, dx, wq, dw, y, nullptr, nullptr, M, N, K, ldc,
                                               0, s);
     case GEMM_ROUTE_BIG:
