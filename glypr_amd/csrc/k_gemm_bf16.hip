@@ -454,9 +454,10 @@ inline bool big_ok(int64_t M, int64_t Nrows, int64_t K) {
 // ---------------------------------------------------------------------------
 // Dense bf16 weights (LinearOp over an F16/BF16 GGUF tensor, linear.rs:48-54,
 // at bf16): C = A . B^T with A bf16 [M][K] and B bf16 [N][K], f32 accumulate.
-// 128 x 128 tiles on a 2 x 2 grid of waves (64 x 64 outputs each, 2 x 2
-// v_mfma_f32_32x32x16_bf16 tiles).  K streams through an LDS ring of RING
-// slots, BKE K per stage (one or two 32-K blocks), A and B each [128 rows]
+// (64 TM) x (64 TN) tiles on a 2 x 2 grid of waves (32 TM x 32 TN outputs each,
+// TM x TN v_mfma_f32_32x32x16_bf16 tiles): 128 x 128, 64 x 128 or 64 x 64 (see
+// run_dense; an output's products and their order are the same in each).  K streams through an LDS ring of RING
+// slots, BKE K per stage (one or two 32-K blocks), A and B each [rows]
 // [2 BKE bytes] by LDS DMA, 16-byte chunk c of row r at c ^ swz(r); the waits
 // count exactly the units issued after each stage, so RING - 1 stages are in
 // flight.  Per 32-K block a lane takes 16 consecutive K of its A row and B
@@ -464,14 +465,13 @@ inline bool big_ok(int64_t M, int64_t Nrows, int64_t K) {
 // GEGLU: 32-row tiles alternate gate and up of the same 32 h columns; h =
 // geglu(gate, up) leaves as bf16.
 // ---------------------------------------------------------------------------
-constexpr int BFW_BM = 128, BFW_BN = 128;
-
-template <bool GEGLU, int BKE, int RING, bool VEC>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
+template <bool GEGLU, int TM, int TN, int BKE, int RING, bool VEC>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RING * (TM + TN) > 10 ? 1 : 2)))
 gemm_bf16w_kernel(const uint16_t* __restrict__ A, const uint16_t* __restrict__ B,
                   float* __restrict__ C, uint16_t* __restrict__ Hb, int M, int N, int K,
                   int ldc, int F, int tiles_n) {
-  constexpr int NW = 4, TM = 2, TN = 2;
+  constexpr int NW = 4, BFW_BM = 64 * TM, BFW_BN = 64 * TN;
+  static_assert(!GEGLU || TN == 2, "a wave's two column tiles are gate and up");
   constexpr int ROWB = 2 * BKE;                 // bytes per LDS row per stage
   constexpr int CPR = ROWB / 16;                // 16-byte chunks per row (4 or 8)
   constexpr int RPU = 1024 / ROWB;              // rows per 1 KB DMA unit
@@ -535,12 +535,12 @@ gemm_bf16w_kernel(const uint16_t* __restrict__ A, const uint16_t* __restrict__ B
       const int q = 4 * p + 2 * lhalf + h;
 #pragma unroll
       for (int tm = 0; tm < TM; tm++) {
-        const int row = 64 * wm + 32 * tm + lrow;
+        const int row = 32 * TM * wm + 32 * tm + lrow;
         offA[tm][p][h] = row * ROWB + ((q ^ swz(row)) << 4);
       }
 #pragma unroll
       for (int tn = 0; tn < TN; tn++) {
-        const int row = 64 * wn + 32 * tn + lrow;
+        const int row = 32 * TN * wn + 32 * tn + lrow;
         offB[tn][p][h] = UA * 1024 + row * ROWB + ((q ^ swz(row)) << 4);
       }
     }
@@ -600,12 +600,12 @@ gemm_bf16w_kernel(const uint16_t* __restrict__ A, const uint16_t* __restrict__ B
     for (int tm = 0; tm < TM; tm++)
 #pragma unroll
       for (int tn = 0; tn < TN; tn++) {
-        const int gn = n0 + 64 * wn + 32 * tn + (VEC ? qc : lrow);
+        const int gn = n0 + 32 * TN * wn + 32 * tn + (VEC ? qc : lrow);
 #pragma unroll
         for (int g = 0; g < 4; g++) {
           float v[4] = {acc[tm][tn][4 * g], acc[tm][tn][4 * g + 1], acc[tm][tn][4 * g + 2],
                         acc[tm][tn][4 * g + 3]};
-          const int gr = m0 + 64 * wm + 32 * tm + 8 * g + 4 * lhalf;
+          const int gr = m0 + 32 * TM * wm + 32 * tm + 8 * g + 4 * lhalf;
           if constexpr (VEC) {
             quad_transpose4(v);
             if (gr + qi < M && gn < N)
@@ -628,7 +628,7 @@ gemm_bf16w_kernel(const uint16_t* __restrict__ A, const uint16_t* __restrict__ B
         float v[4];
 #pragma unroll
         for (int j = 0; j < 4; j++) v[j] = geglu_bf16(acc[tm][0][4 * g + j], acc[tm][1][4 * g + j]);
-        const int gr = m0 + 64 * wm + 32 * tm + 8 * g + 4 * lhalf;
+        const int gr = m0 + 32 * TM * wm + 32 * tm + 8 * g + 4 * lhalf;
         if constexpr (VEC) {
           quad_transpose4(v);
           const uint32_t lo = __builtin_bit_cast(uint16_t, (__bf16)v[0]) |
@@ -794,21 +794,43 @@ gemm_bf16w_qkv_kernel(const uint16_t* __restrict__ A, const uint16_t* __restrict
   }
 }
 
-template <bool GEGLU>
-hipError_t run_dense(const uint16_t* xb, const uint16_t* wb, float* y, uint16_t* hb, int64_t M,
-                     int64_t Nrows, int64_t K, int64_t ldc, int64_t F, hipStream_t s) {
-  const int64_t tiles_n = (Nrows + BFW_BN - 1) / BFW_BN;
-  const int64_t tiles = ((M + BFW_BM - 1) / BFW_BM) * tiles_n;
+template <bool GEGLU, int TM, int TN, int RING>
+hipError_t run_dense_tile(const uint16_t* xb, const uint16_t* wb, float* y, uint16_t* hb,
+                          int64_t M, int64_t Nrows, int64_t K, int64_t ldc, int64_t F,
+                          hipStream_t s) {
+  constexpr int BM = 64 * TM, BN = 64 * TN;
+  const int64_t tiles_n = (Nrows + BN - 1) / BN;
+  const int64_t tiles = ((M + BM - 1) / BM) * tiles_n;
   const bool vec = GEGLU ? F % 4 == 0 && (reinterpret_cast<uintptr_t>(hb) & 7) == 0
                          : Nrows % 4 == 0 && ldc % 4 == 0 &&
                                (reinterpret_cast<uintptr_t>(y) & 15) == 0;
   if (vec)
-    gemm_bf16w_kernel<GEGLU, 64, 2, true><<<dim3((unsigned)tiles), 256, 0, s>>>(
+    gemm_bf16w_kernel<GEGLU, TM, TN, 64, RING, true><<<dim3((unsigned)tiles), 256, 0, s>>>(
         xb, wb, y, hb, (int)M, (int)Nrows, (int)K, (int)ldc, (int)F, (int)tiles_n);
   else
-    gemm_bf16w_kernel<GEGLU, 64, 2, false><<<dim3((unsigned)tiles), 256, 0, s>>>(
+    gemm_bf16w_kernel<GEGLU, TM, TN, 64, RING, false><<<dim3((unsigned)tiles), 256, 0, s>>>(
         xb, wb, y, hb, (int)M, (int)Nrows, (int)K, (int)ldc, (int)F, (int)tiles_n);
   return hipGetLastError();
+}
+
+// The plain GEMM's tile.  Up to 640 tiles of 64 x 64 (2.5 per CU) the 128 x 128
+// grid leaves most CUs idle and each workgroup alone with its DMA latency:
+// 64 x 64 tiles on a three-slot ring (300 x 1152 x 768: 13.7 -> 6.7 us; 1000 x
+// 2048 x 512: 21.0 -> 9.6; 3001 x 1152 x 768: 15.6 -> 13.5).  Above, 64 x 128
+// tiles (three workgroups per CU) where 128 x 128 ones fill at most one per CU
+// or N is below 2048 (8192 x 768 x 1280: 29.5 -> 27.0; 16384: 54.4 -> 48.7);
+// 5000 x 768 x 2304 stays at 128 x 128 (29.5 against 32.7), which reads a third
+// less LDS per product.
+template <bool GEGLU>
+hipError_t run_dense(const uint16_t* xb, const uint16_t* wb, float* y, uint16_t* hb, int64_t M,
+                     int64_t Nrows, int64_t K, int64_t ldc, int64_t F, hipStream_t s) {
+  if constexpr (!GEGLU) {
+    if (((M + 63) / 64) * ((Nrows + 63) / 64) <= 640)
+      return run_dense_tile<false, 1, 1, 3>(xb, wb, y, hb, M, Nrows, K, ldc, F, s);
+    if (Nrows < 2048 || ((M + 127) / 128) * ((Nrows + 127) / 128) <= 256)
+      return run_dense_tile<false, 1, 2, 2>(xb, wb, y, hb, M, Nrows, K, ldc, F, s);
+  }
+  return run_dense_tile<GEGLU, 2, 2, 2>(xb, wb, y, hb, M, Nrows, K, ldc, F, s);
 }
 
 }  // namespace
