@@ -23,11 +23,18 @@ __all__ = ["Context", "Q8Weight", "BF16Weight", "INT8_EXACT", "BF16_DEQUANT", "I
 
 
 def _ptr(t: Optional[torch.Tensor]):
+    """The tensor's address, an int that ctypes passes as void* (no c_void_p object)."""
     if t is None:
         return None
     if not t.is_contiguous():
         raise ValueError("tensor must be contiguous")
-    return ctypes.c_void_p(t.data_ptr())
+    return t.data_ptr()
+
+
+# The current stream's handle without a torch.cuda.Stream object around it (0.08
+# against 1.1 us, a seventh of a small call); the public property where torch has
+# no such function, and before CUDA is initialised (it initialises it).
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 
 
 class Context:
@@ -41,10 +48,17 @@ class Context:
 
     @property
     def stream(self):
-        return ctypes.c_void_p(torch.cuda.current_stream(self.device).cuda_stream)
+        return ctypes.c_void_p(self._stream)
+
+    @property
+    def _stream(self) -> int:
+        """The current stream's handle on the context's device."""
+        if _raw_stream is not None and torch.cuda.is_initialized():
+            return _raw_stream(self.device)
+        return torch.cuda.current_stream(self.device).cuda_stream
 
     def sync(self):
-        check(lib().glypr_hip_sync(self.handle, self.stream))
+        check(lib().glypr_hip_sync(self.handle, self._stream))
 
     def reserve(self, rows: int):
         """glypr_hip_ctx_reserve: size the workspace for `rows` activation rows."""
@@ -62,7 +76,7 @@ class Context:
             pass
 
     def _check_tensor(self, t: torch.Tensor, name: str, dtype=torch.float32):
-        if t.device.type != "cuda" or t.device.index != self.device:
+        if not t.is_cuda or t.get_device() != self.device:
             raise ValueError(f"{name} must be on cuda:{self.device}")
         if t.dtype != dtype:
             raise ValueError(f"{name} must be {dtype}")
@@ -164,14 +178,12 @@ def bf16_matmul(ctx: Context, w: BF16Weight, x: torch.Tensor,
     ctx._check_tensor(x, "x")
     m = x.numel() // w.k
     y = _out(x, (*x.shape[:-1], w.n), out)
-    check(lib().glypr_hip_bf16_matmul(ctx.handle, w.handle, _ptr(x), _ptr(y), m, ctx.stream))
+    check(lib().glypr_hip_bf16_matmul(ctx.handle, w.handle, _ptr(x), _ptr(y), m, ctx._stream))
     return y
 
 
 def _out(x: torch.Tensor, shape, out: Optional[torch.Tensor]):
-    if out is None:
-        return torch.empty(shape, dtype=torch.float32, device=x.device)
-    return out
+    return x.new_empty(shape) if out is None else out   # x is f32 (_check_tensor)
 
 
 def q8_0_matmul(ctx: Context, w: Q8Weight, x: torch.Tensor, variant: int = INT8_EXACT,
@@ -180,7 +192,7 @@ def q8_0_matmul(ctx: Context, w: Q8Weight, x: torch.Tensor, variant: int = INT8_
     m = x.numel() // w.k
     y = _out(x, (*x.shape[:-1], w.n), out)
     check(lib().glypr_hip_q8_0_matmul(ctx.handle, w.handle, _ptr(x), _ptr(y), m, variant,
-                                      ctx.stream))
+                                      ctx._stream))
     return y
 
 
@@ -192,7 +204,7 @@ def q8_0_matmul_noalloc(ctx: Context, w: Q8Weight, x: torch.Tensor, variant: int
     m = x.numel() // w.k
     y = _out(x, (*x.shape[:-1], w.n), out)
     check(lib().glypr_hip_q8_0_matmul_noalloc(ctx.handle, w.handle, _ptr(x), _ptr(y), m, variant,
-                                              ctx.stream))
+                                              ctx._stream))
     return y
 
 
@@ -204,7 +216,7 @@ def rmsnorm_q8_0_matmul(ctx: Context, w: Q8Weight, x: torch.Tensor,
     m = x.numel() // w.k
     y = _out(x, (*x.shape[:-1], w.n), out)
     check(lib().glypr_hip_rmsnorm_q8_0_matmul(ctx.handle, w.handle, _ptr(x), _ptr(norm_weight),
-                                              eps, _ptr(y), m, variant, ctx.stream))
+                                              eps, _ptr(y), m, variant, ctx._stream))
     return y
 
 
@@ -214,7 +226,7 @@ def rmsnorm(ctx: Context, x: torch.Tensor, weight: Optional[torch.Tensor], eps: 
     d = x.shape[-1]
     y = _out(x, x.shape, out)
     check(lib().glypr_hip_rmsnorm(ctx.handle, _ptr(x), _ptr(weight), eps, _ptr(y),
-                                  x.numel() // d, d, ctx.stream))
+                                  x.numel() // d, d, ctx._stream))
     return y
 
 
@@ -226,7 +238,7 @@ def geglu(ctx: Context, gate: torch.Tensor, up: torch.Tensor,
         raise ValueError("gate/up shape mismatch")
     y = _out(gate, gate.shape, out)
     check(lib().glypr_hip_geglu(ctx.handle, _ptr(gate), _ptr(up), _ptr(y), gate.numel(),
-                                ctx.stream))
+                                ctx._stream))
     return y
 
 
@@ -236,7 +248,7 @@ def mlp(ctx: Context, gate_up: Q8Weight, down: Q8Weight, x: torch.Tensor,
     m = x.numel() // gate_up.k
     y = _out(x, (*x.shape[:-1], down.n), out)
     check(lib().glypr_hip_mlp(ctx.handle, gate_up.handle, down.handle, _ptr(x), _ptr(y), m,
-                              variant, ctx.stream))
+                              variant, ctx._stream))
     return y
 
 
@@ -247,13 +259,13 @@ def rmsnorm_mlp(ctx: Context, gate_up: Q8Weight, down: Q8Weight, x: torch.Tensor
     m = x.numel() // gate_up.k
     y = _out(x, (*x.shape[:-1], down.n), out)
     check(lib().glypr_hip_rmsnorm_mlp(ctx.handle, gate_up.handle, down.handle, _ptr(x),
-                                      _ptr(norm_weight), eps, _ptr(y), m, variant, ctx.stream))
+                                      _ptr(norm_weight), eps, _ptr(y), m, variant, ctx._stream))
     return y
 
 
 def dequantize(ctx: Context, w: Q8Weight) -> torch.Tensor:
     y = torch.empty((w.n, w.k), dtype=torch.float32, device=f"cuda:{ctx.device}")
-    check(lib().glypr_hip_q8_0_dequantize(ctx.handle, w.handle, _ptr(y), ctx.stream))
+    check(lib().glypr_hip_q8_0_dequantize(ctx.handle, w.handle, _ptr(y), ctx._stream))
     return y
 
 
@@ -261,8 +273,8 @@ def quantize(ctx: Context, x: torch.Tensor) -> torch.Tensor:
     ctx._check_tensor(x, "x")
     k = x.shape[-1]
     m = x.numel() // k
-    out = torch.empty((m, k // 32 * 34), dtype=torch.uint8, device=x.device)
-    check(lib().glypr_hip_q8_0_quantize(ctx.handle, _ptr(x), m, k, _ptr(out), ctx.stream))
+    out = x.new_empty((m, k // 32 * 34), dtype=torch.uint8)
+    check(lib().glypr_hip_q8_0_quantize(ctx.handle, _ptr(x), m, k, _ptr(out), ctx._stream))
     return out
 
 
@@ -273,7 +285,7 @@ def embed_gather(ctx: Context, table: Q8Weight, ids, scale: float,
         out = torch.empty((ids.size, table.k), dtype=torch.float32, device=f"cuda:{ctx.device}")
     check(lib().glypr_hip_q8_0_embed_gather(ctx.handle, table.handle,
                                             ids.ctypes.data_as(ctypes.c_void_p), ids.size,
-                                            scale, _ptr(out), ctx.stream))
+                                            scale, _ptr(out), ctx._stream))
     return out
 
 
@@ -290,7 +302,7 @@ def pool_normalize(ctx: Context, tokens: torch.Tensor, mask=None, trunc: int = 0
     check(lib().glypr_hip_pool_normalize(
         ctx.handle, _ptr(tokens),
         None if mk is None else mk.ctypes.data_as(ctypes.c_void_p), t, d, trunc, _ptr(out),
-        ctx.stream))
+        ctx._stream))
     return out
 
 
@@ -304,8 +316,8 @@ def quantize_binary(ctx: Context, x: torch.Tensor, out: Optional[torch.Tensor] =
     ctx._check_tensor(x, "x")
     n, dim = x.shape
     if out is None:
-        out = torch.empty((n, dim // 64), dtype=torch.int64, device=x.device)
-    check(lib().glypr_hip_quantize_binary(ctx.handle, _ptr(x), n, dim, _ptr(out), ctx.stream))
+        out = x.new_empty((n, dim // 64), dtype=torch.int64)
+    check(lib().glypr_hip_quantize_binary(ctx.handle, _ptr(x), n, dim, _ptr(out), ctx._stream))
     return out
 
 
@@ -314,8 +326,8 @@ def quantize_int8(ctx: Context, x: torch.Tensor, out: Optional[torch.Tensor] = N
     """quantize_int8 (util.rs:128-133), elementwise."""
     ctx._check_tensor(x, "x")
     if out is None:
-        out = torch.empty(x.shape, dtype=torch.int8, device=x.device)
-    check(lib().glypr_hip_quantize_int8(ctx.handle, _ptr(x), x.numel(), _ptr(out), ctx.stream))
+        out = x.new_empty(x.shape, dtype=torch.int8)
+    check(lib().glypr_hip_quantize_int8(ctx.handle, _ptr(x), x.numel(), _ptr(out), ctx._stream))
     return out
 
 
@@ -330,36 +342,36 @@ def _pairs(ctx: Context, a: torch.Tensor, b: torch.Tensor, dtype, name: str):
 def hamming(ctx: Context, a: torch.Tensor, b: torch.Tensor) -> torch.Tensor:
     """hamming_distance (util.rs:75-109) for all pairs -> int32 [na, nb]."""
     na, nb, w = _pairs(ctx, a, b, torch.int64, "hamming")
-    out = torch.empty((na, nb), dtype=torch.int32, device=a.device)
+    out = a.new_empty((na, nb), dtype=torch.int32)
     check(lib().glypr_hip_hamming(ctx.handle, _ptr(a), na, _ptr(b), nb, w, _ptr(out),
-                                  ctx.stream))
+                                  ctx._stream))
     return out
 
 
 def binary_cosine(ctx: Context, a: torch.Tensor, b: torch.Tensor) -> torch.Tensor:
     """binary_cosine_similarity (util.rs:112-119) for all pairs -> f32 [na, nb]."""
     na, nb, w = _pairs(ctx, a, b, torch.int64, "binary_cosine")
-    out = torch.empty((na, nb), dtype=torch.float32, device=a.device)
+    out = a.new_empty((na, nb), dtype=torch.float32)
     check(lib().glypr_hip_binary_cosine(ctx.handle, _ptr(a), na, _ptr(b), nb, w, _ptr(out),
-                                        ctx.stream))
+                                        ctx._stream))
     return out
 
 
 def int8_dot(ctx: Context, a: torch.Tensor, b: torch.Tensor) -> torch.Tensor:
     """int8_dot_product (util.rs:137-176) for all pairs -> int32 [na, nb]."""
     na, nb, d = _pairs(ctx, a, b, torch.int8, "int8_dot")
-    out = torch.empty((na, nb), dtype=torch.int32, device=a.device)
+    out = a.new_empty((na, nb), dtype=torch.int32)
     check(lib().glypr_hip_int8_dot(ctx.handle, _ptr(a), na, _ptr(b), nb, d, _ptr(out),
-                                   ctx.stream))
+                                   ctx._stream))
     return out
 
 
 def int8_cosine(ctx: Context, a: torch.Tensor, b: torch.Tensor) -> torch.Tensor:
     """int8_cosine_similarity (util.rs:181-197) for all pairs -> f32 [na, nb]."""
     na, nb, d = _pairs(ctx, a, b, torch.int8, "int8_cosine")
-    out = torch.empty((na, nb), dtype=torch.float32, device=a.device)
+    out = a.new_empty((na, nb), dtype=torch.float32)
     check(lib().glypr_hip_int8_cosine(ctx.handle, _ptr(a), na, _ptr(b), nb, d, _ptr(out),
-                                      ctx.stream))
+                                      ctx._stream))
     return out
 
 
@@ -373,7 +385,7 @@ def attention(ctx: Context, qkv: torch.Tensor, q_norm: torch.Tensor, k_norm: tor
     y = _out(qkv, (t, n_heads * head_dim), out)
     check(lib().glypr_hip_attention(ctx.handle, _ptr(qkv), _ptr(q_norm), _ptr(k_norm), eps,
                                     _ptr(cos_t), _ptr(sin_t), t, n_heads, n_kv_heads, head_dim,
-                                    window, _ptr(y), ctx.stream))
+                                    window, _ptr(y), ctx._stream))
     return y
 
 
@@ -540,7 +552,7 @@ class Model:
             out = torch.empty(td, dtype=torch.float32, device=f"cuda:{self.ctx.device}")
         check(lib().glypr_hip_model_embed(self.handle, ids.ctypes.data_as(ctypes.c_void_p),
                                           ids.size, trunc, _ptr(out), _ptr(hidden),
-                                          self.ctx.stream))
+                                          self.ctx._stream))
         return out
 
     def embed_batch(self, seqs, trunc: int = 0, out: Optional[torch.Tensor] = None):
@@ -555,7 +567,7 @@ class Model:
                               device=f"cuda:{self.ctx.device}")
         check(lib().glypr_hip_model_embed_batch(self.handle, ids.ctypes.data_as(ctypes.c_void_p),
                                                 lens.ctypes.data_as(ctypes.c_void_p), len(seqs),
-                                                trunc, _ptr(out), self.ctx.stream))
+                                                trunc, _ptr(out), self.ctx._stream))
         return out
 
     def close(self):
