@@ -224,11 +224,12 @@ hipError_t run(const uint16_t* xb, const int8_t* wq, const float* dw, float* y, 
 }
 
 // ---------------------------------------------------------------------------
-// Large-M variant (M > 2048, K % 64 == 0).  128 x 128 tiles on 4 waves side
-// by side along N, 128 x 32 outputs each (4 v_mfma_f32_32x32x16_bf16 tiles
-// stacked along M), so every B column is dequantized by exactly one wave;
-// every 64-K stage arrives by LDS DMA into a two-slot ring:
-//   A  [128 rows][128 B] bf16, 16-byte chunk c of row r at c ^ ((r >> 1) & 7);
+// LDS-DMA variant (K % 64 == 0).  32 TM x 128 tiles (TM = 1, 2, 4; see
+// run_big_rows) on 4 waves side by side along N, 32 TM x 32 outputs each (TM
+// v_mfma_f32_32x32x16_bf16 tiles stacked along M), so every B column is
+// dequantized by exactly one wave; every 64-K stage arrives by LDS DMA into a
+// two-slot ring:
+//   A  [32 TM rows][128 B] bf16, 16-byte chunk c of row r at c ^ ((r >> 1) & 7);
 //   B  [128 rows][64 B]  int8, chunk c of row r at c ^ ((r >> 2) & 3);
 //   dB [2 blocks][128 rows] f32.
 // Per 32-K block a lane reads 16 consecutive K of its A row (two b128) and
@@ -236,8 +237,8 @@ hipError_t run(const uint16_t* xb, const int8_t* wq, const float* dw, float* y, 
 // (dequant16: the exact q*d, then bf16 round-to-nearest-even, as the staged
 // path) and runs two MFMA k-steps on K {0..7, 16..23} and {8..15, 24..31} of
 // the block; A and B use the same order, so every product is formed once.
-// XCD-aware tile order as in the int8 large-M kernel; 50 KB of LDS and ~120
-// VGPRs, so three workgroups share a CU.  The 128-column tile (rather than
+// XCD-aware tile order as in the int8 large-M kernel; at TM = 4 50 KB of LDS and
+// ~120 VGPRs, so three workgroups share a CU.  The 128-column tile (rather than
 // 256) keeps the grids of the C3 projections near whole rounds of 768
 // workgroup slots.
 // GEGLU: the 32 B rows of wave w are gate columns hc0 + 16 w .. + 15, then
@@ -445,9 +446,27 @@ hipError_t run_big(const uint16_t* xb, const int8_t* wq, const float* dw, float*
   return hipGetLastError();
 }
 
-// The large-M kernel addresses operands with 32-bit offsets.
+// Rows per workgroup: 32 or 64 while such tiles do not fill the CUs (a tile's
+// time is its K stages' DMA latency then, whatever its height), else 128.
+// Against the register-staged kernel that took M <= 2048, 300 x 768 x 1280 10.3
+// -> 8.6 us, 1000 x 2048 x 512 23.5 -> 18.6, 2048 x 768 x 1280 15.2 -> 11.3, gate/up
+// 1000 x 512 x 4096 15.8 -> 10.4; against 128 rows, 2500 x 768 x 768 11.6 -> 10.4
+// (4800 x 768 x 1280 stays: 16.6 against 17.9).
+template <bool GEGLU>
+hipError_t run_big_rows(const uint16_t* xb, const int8_t* wq, const float* dw, float* y,
+                        uint16_t* hb, int64_t M, int64_t Nrows, int64_t K, int64_t ldc, int64_t F,
+                        hipStream_t s) {
+  const int64_t tiles_n = (Nrows + BFB_BN - 1) / BFB_BN;
+  if ((M + 31) / 32 * tiles_n <= 256)
+    return run_big<GEGLU, 1>(xb, wq, dw, y, hb, M, Nrows, K, ldc, F, s);
+  if (M <= 2048 || (M + 63) / 64 * tiles_n <= 384)
+    return run_big<GEGLU, 2>(xb, wq, dw, y, hb, M, Nrows, K, ldc, F, s);
+  return run_big<GEGLU, 4>(xb, wq, dw, y, hb, M, Nrows, K, ldc, F, s);
+}
+
+// The LDS-DMA kernel addresses operands with 32-bit offsets.
 inline bool big_ok(int64_t M, int64_t Nrows, int64_t K) {
-  return M > 2048 && K % BFB_BK == 0 && 2 * M * K < (int64_t(1) << 31) &&
+  return K % BFB_BK == 0 && 2 * M * K < (int64_t(1) << 31) &&
          Nrows * K < (int64_t(1) << 31);
 }
 
@@ -838,7 +857,7 @@ hipError_t run_dense(const uint16_t* xb, const uint16_t* wb, float* y, uint16_t*
 hipError_t launch_gemm_bf16(const uint16_t* xb, const int8_t* wq, const float* dw, float* y,
                             int64_t M, int64_t N, int64_t K, int64_t ldc, hipStream_t s) {
   if (M == 0 || N == 0) return hipSuccess;
-  if (big_ok(M, N, K)) return run_big<false, 4>(xb, wq, dw, y, nullptr, M, N, K, ldc, 0, s);
+  if (big_ok(M, N, K)) return run_big_rows<false>(xb, wq, dw, y, nullptr, M, N, K, ldc, 0, s);
   int64_t big_tiles = ((M + 255) / 256) * ((N + 127) / 128);
   if (big_tiles >= 256)
     return run<256, 128, 4, 2, false>(xb, wq, dw, y, nullptr, M, N, K, ldc, 0, s);
@@ -848,7 +867,7 @@ hipError_t launch_gemm_bf16(const uint16_t* xb, const int8_t* wq, const float* d
 hipError_t launch_gemm_bf16_geglu(const uint16_t* xb, const int8_t* wq, const float* dw,
                                   uint16_t* hb, int64_t M, int64_t F, int64_t K, hipStream_t s) {
   if (M == 0 || F == 0) return hipSuccess;
-  if (big_ok(M, 2 * F, K)) return run_big<true, 4>(xb, wq, dw, nullptr, hb, M, 2 * F, K, 0, F, s);
+  if (big_ok(M, 2 * F, K)) return run_big_rows<true>(xb, wq, dw, nullptr, hb, M, 2 * F, K, 0, F, s);
   int64_t big_tiles = ((M + 255) / 256) * ((2 * F + 127) / 128);
   if (big_tiles >= 256)
     return run<256, 128, 4, 2, true>(xb, wq, dw, nullptr, hb, M, 2 * F, K, 0, F, s);
