@@ -54,12 +54,27 @@ __device__ __forceinline__ float max8(float v) {
 // max8 for values that are >= +0 and never NaN (block amax of |x|, which
 // starts from 0 and ignores NaN like Rust's f32::max): their bit patterns
 // order like the floats, so the reduction is an integer max.
+// umax_dpp: max with the DPP-permuted self, one v_max_u32_dpp (every lane has
+// a source under the controls used here, so the zero fill is never taken; it
+// is what lets the compiler fold the move into the max).
+template <int CTRL>
+__device__ __forceinline__ uint32_t umax_dpp(uint32_t u) {
+  return max(u, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)u, CTRL, 0xF, 0xF, true));
+}
+__device__ __forceinline__ uint32_t umax8(uint32_t u) {
+  u = umax_dpp<0xB1>(u);     // quad_perm [1,0,3,2]
+  u = umax_dpp<0x4E>(u);     // quad_perm [2,3,0,1]
+  return umax_dpp<0x141>(u);  // row_half_mirror: quad 0 <-> quad 1
+}
 __device__ __forceinline__ float max8_nonneg(float v) {
-  uint32_t u = __float_as_uint(v);
-  u = max(u, (uint32_t)__builtin_amdgcn_update_dpp((int)u, (int)u, 0xB1, 0xF, 0xF, false));
-  u = max(u, (uint32_t)__builtin_amdgcn_update_dpp((int)u, (int)u, 0x4E, 0xF, 0xF, false));
-  u = max(u, (uint32_t)__builtin_amdgcn_update_dpp((int)u, (int)u, 0x141, 0xF, 0xF, false));
-  return __uint_as_float(u);
+  return __uint_as_float(umax8(__float_as_uint(v)));
+}
+// |h| as ordered bits, NaN -> 0 (an amax starts from 0 and skips NaN); one
+// instruction, where fmaxf(0, fabsf(h)) also quiets its operand
+__device__ __forceinline__ uint32_t abs_bits_no_nan(float h) {
+  uint32_t u;
+  asm("v_max_f32_e64 %0, 0, |%1|" : "=v"(u) : "v"(h));
+  return u;
 }
 // v of lane I of each aligned group of 8 lanes, to every lane of the group
 // (ds_swizzle bit mode: lane' = (lane & 0x18) | I within each 32 lanes).
@@ -82,9 +97,7 @@ __device__ __forceinline__ float bcast8(float v, int i) {
 }
 // max16 for values that are >= +0 and never NaN (see max8_nonneg)
 __device__ __forceinline__ float max16_nonneg(float v) {
-  uint32_t u = __float_as_uint(max8_nonneg(v));
-  u = max(u, (uint32_t)__builtin_amdgcn_update_dpp((int)u, (int)u, 0x140, 0xF, 0xF, false));
-  return __uint_as_float(u);
+  return __uint_as_float(umax_dpp<0x140>(umax8(__float_as_uint(v))));   // row_mirror
 }
 // v of lane I of each aligned group of 16 lanes, to every lane of the group
 template <int I>
@@ -307,16 +320,29 @@ __device__ __forceinline__ float expm1_nonpos(float y) {
   return fmaf(sc, p, sc - 1.0f);
 }
 
+// -t / (t + 2) correctly rounded, for t in [-1, -2^-12]: the operands need no
+// scaling, so Newton's step on the reciprocal and one residual correction of
+// the quotient (Markstein) replace the general division's scale and fix-up
+// instructions: 6 in place of 11.  Equal to the IEEE quotient for every float
+// of the range (all 10^8 compared on gfx950).
+__device__ __forceinline__ float tanh_quotient(float t) {
+  const float d = t + 2.0f, n = -t;
+  float r = __builtin_amdgcn_rcpf(d);
+  r = fmaf(fmaf(-d, r, 1.0f), r, r);
+  const float q = n * r;
+  return fmaf(fmaf(-d, q, n), r, q);
+}
+
 // orc_tanhf's value for every input.  The general path runs on |x| clamped to
 // [2^-12, 10]: at 10 it gives expm1(-20) = -1.0f exactly and so +-1, which is
-// orc_tanhf's |x| >= 10 result; the NaN and |x| < 2^-12 cases (-> x) are
-// selects.
+// orc_tanhf's |x| >= 10 result; the NaN and |x| < 2^-12 cases (-> x) are one
+// select (an unordered compare fails).
 __device__ __forceinline__ float tanh_glypr(float x) {
   const float ax = fabsf(x);
-  const float axc = fminf(fmaxf(ax, 2.44140625e-04f), 10.0f);
+  const float axc = __builtin_amdgcn_fmed3f(ax, 2.44140625e-04f, 10.0f);
   const float t = expm1_nonpos(-2.0f * axc);
-  const float r = materialize(copysignf(-t / (t + 2.0f), x));
-  return (x != x || ax < 2.44140625e-04f) ? x : r;
+  const float r = materialize(copysignf(tanh_quotient(t), x));
+  return ax >= 2.44140625e-04f ? r : x;
 }
 
 // geglu_scalar_f32 (cpu_simd/geglu.rs:6-18).  For g >= 10 the general path

@@ -1068,6 +1068,11 @@ hipError_t run_pro(const float* x, const float* nw, float eps, const int8_t* wq,
 // up c+32..c+63], so a Q8_0 block of h is one MFMA tile pair: the block amax
 // is a 32-lane reduction, and each wave derives its 64 (row, block) scales one
 // per lane through a per-wave LDS table instead of repeating the divisions.
+// The epilogue is VALU time on top of the blocks' (~55 instructions per h
+// element; ~95 with a DPP move, a quieting max and a max per reduction level,
+// byte stores and a general division in tanh): 8190 x 512 -> 2 x 2048 99 -> 83 us,
+// 16384 x 768 -> 2 x 1152 138 -> 123.  64 x 128, 128 x 64 and 64 x 64 tiles are
+// slower at 8190 (91 to 96 us) and equal at 4800 x 768 -> 2 x 1152 (46 to 48).
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ int big_swz(int row) { return (row >> 1) & 7; }
 
@@ -1219,47 +1224,82 @@ gemm_i8_big_kernel(const int8_t* __restrict__ A, const float* __restrict__ dA,
     }
   } else {
     // h block p (columns c + 32 p .. +31) of row (r, lhalf) is lane lrow's
-    // value of geglu(acc[2p][r], acc[2p+1][r]).  Scale table per wave in the
-    // ring slot of stage nst - 2, which every wave finished before the last
-    // barrier: amax[lhalf][p][r], then (id, dq) per entry.
-    constexpr int TE = 16 * TN;   // table entries: (lhalf, p, r)
-    static_assert(TN % 2 == 0, "gate and up tiles in pairs");
+    // value of geglu(acc[2p][r], acc[2p+1][r]).  Block amax: v_permlane16_swap
+    // puts registers 2j and 2j + 1 side by side in the 16-lane rows, so one max
+    // covers both, and four DPP maxima finish the pair (48 instructions for 16
+    // registers against 5 x 4 per register of 32-lane shuffled maxima).  Table
+    // per wave in the ring slot of stage nst - 2, which every wave finished
+    // before the last barrier: entry [lhalf][r & 1][p][r >> 1], whose scale one
+    // lane derives and stores.  The int8 rows leave as dwords: a 4 x 4 byte
+    // transpose inside each quad of lanes turns four rows' bytes of one column
+    // into four columns of one row.
+    constexpr int NP = TN / 2, TE = 32 * NP;   // table entries
+    static_assert(TN % 2 == 0 && TE <= 64, "gate and up tiles in pairs, one entry per lane");
     const int nbh = F / QK;
-    float* tab = reinterpret_cast<float*>(ring + (((nst - 1) & 1) ^ 1) * SLOT) + wave * TE * 3;
-    float h[TN / 2][16];
+    uint32_t* tab =
+        reinterpret_cast<uint32_t*>(ring + (((nst - 1) & 1) ^ 1) * SLOT) + wave * TE * 2;
+    float h[NP][16];
+    uint32_t am[NP][8];
 #pragma unroll
-    for (int p = 0; p < TN / 2; p++)
+    for (int p = 0; p < NP; p++)
 #pragma unroll
-      for (int r = 0; r < 16; r++) {
-        h[p][r] = geglu_scalar(acc[2 * p][r], acc[2 * p + 1][r]);
-        const float v = max32_hi(fmaxf(0.0f, fabsf(h[p][r])));
-        if (lrow == 31) tab[lhalf * (TE / 2) + p * 16 + r] = v;
+      for (int j = 0; j < 8; j++) {
+        h[p][2 * j] = geglu_scalar(acc[2 * p][2 * j], acc[2 * p + 1][2 * j]);
+        h[p][2 * j + 1] = geglu_scalar(acc[2 * p][2 * j + 1], acc[2 * p + 1][2 * j + 1]);
+        const auto sw = __builtin_amdgcn_permlane16_swap(abs_bits_no_nan(h[p][2 * j]),
+                                                         abs_bits_no_nan(h[p][2 * j + 1]), false,
+                                                         false);
+        am[p][j] = umax_dpp<0x140>(umax8(max(sw[0], sw[1])));   // row_mirror last
       }
+    if ((lane & 15) == 0) {
+      uint4* t4 = reinterpret_cast<uint4*>(tab + (lane >> 4) * 8 * NP);
+#pragma unroll
+      for (int p = 0; p < NP; p++)
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+          t4[2 * p + i] = make_uint4(am[p][4 * i], am[p][4 * i + 1], am[p][4 * i + 2],
+                                     am[p][4 * i + 3]);
+    }
     // LDS serves a wave's accesses in order; the fences keep the compiler
     // from moving the table accesses across each other.
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    const int c = hc0 + wn * 16 * TN;
     if (TE >= 64 || lane < TE) {
-      const QScale q = q8_scale(tab[lane]);
-      tab[TE + lane] = q.id;
-      tab[2 * TE + lane] = q.dq;
+      const QScale q = q8_scale(__uint_as_float(tab[lane]));
+      tab[TE + lane] = __float_as_uint(q.id);
+      const int e_half = lane / (16 * NP), e_p = (lane >> 3) & (NP - 1);
+      const int r = 2 * (lane & 7) + ((lane / (8 * NP)) & 1);
+      const int gm = m0 + wm * 32 + 4 * e_half + 8 * (r >> 2) + (r & 3), hb = c + 32 * e_p;
+      if (gm < M && hb < F) dH[(int64_t)gm * nbh + (hb >> 5)] = q.dq;
     }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    const int c = hc0 + wn * 16 * TN;
+    const float* ids = reinterpret_cast<const float*>(tab + TE) + lhalf * 16 * NP;
+    // byte selectors of the transpose: odd lanes of a pair keep the partner's
+    // odd bytes, the upper pair of a quad the other pair's upper half
+    const uint32_t sel0 = (lane & 1) ? 0x03070105u : 0x06020400u;
+    const uint32_t sel1 = (lane & 2) ? 0x03020706u : 0x05040100u;
 #pragma unroll
-    for (int p = 0; p < TN / 2; p++) {
+    for (int p = 0; p < NP; p++) {
       const int hb = c + 32 * p;   // first column of the h block
 #pragma unroll
-      for (int r = 0; r < 16; r++) {
-        const int gm = row0 + 8 * (r >> 2) + (r & 3);
-        const int e = lhalf * (TE / 2) + p * 16 + r;
-        if (gm < M && hb < F) {
-          Hq[(int64_t)gm * F + hb + lrow] = (int8_t)quant_round(h[p][r] * tab[TE + e]);
-          if (lrow == 0) dH[(int64_t)gm * nbh + (hb >> 5)] = tab[2 * TE + e];
-        }
+      for (int g = 0; g < 4; g++) {   // rows 8 g + 4 lhalf + 0 .. 3
+        uint32_t b[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+          b[i] = (uint32_t)quant_round(h[p][4 * g + i] * ids[(i & 1) * 8 * NP + p * 8 + 2 * g + (i >> 1)]);
+        const uint32_t w = __builtin_amdgcn_perm(b[1], b[0], 0x0c0c0400u) |
+                           __builtin_amdgcn_perm(b[3], b[2], 0x04000c0cu);
+        const uint32_t w1 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)w, 0xB1, 0xF, 0xF, true);
+        const uint32_t v = __builtin_amdgcn_perm(w1, w, sel0);
+        const uint32_t v1 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x4E, 0xF, 0xF, true);
+        const uint32_t o = __builtin_amdgcn_perm(v1, v, sel1);
+        const int gm = row0 + 8 * g + (lane & 3);
+        if (gm < M && hb < F)
+          *reinterpret_cast<uint32_t*>(Hq + (int64_t)gm * F + hb + (lrow & ~3)) = o;
       }
     }
   }

@@ -29,3 +29,29 @@ def test_matmul_tiles_bit_exact(ctx, oracle, m, k, n):
     assert_bits_equal(y[rows], oracle.matmul(x[rows], wb, n), f"{m}x{k}x{n}")
     f = host(ops.q8_0_matmul(ctx, w, dev(x), INT8_FMA))
     assert_bits_equal(f[rows], oracle.matmul_fma(x[rows], wb, n), f"fma {m}x{k}x{n}")
+
+
+@pytest.mark.parametrize("m,H,F,scale", [(2049, 128, 32, 1.0), (2113, 256, 96, 8.0),
+                                         (2177, 128, 160, 64.0), (2307, 256, 64, 1e-3)])
+def test_geglu_tile_epilogue_bit_exact(ctx, oracle, m, H, F, scale):
+    """The 128 x 128 tile's GeGLU epilogue: one h block to a partial pair, gates
+    from the tanh's linear range to its saturation, rows of zeros, of single
+    values, and of infinities and NaN."""
+    say(f"geglu epilogue m={m} H={H} F={F} scale={scale}")
+    x = (oracle.normal(m * H, seed=700 + m).reshape(m, H) * scale).astype(np.float32)
+    x[5] = 0
+    x[40] = 0
+    x[40, 7] = 3 * scale
+    x[66] *= np.float32(1e30)
+    x[67] *= np.float32(1e-30)
+    x[90, 3] = np.inf
+    x[91, 3] = np.nan
+    gb, ub, db = (oracle.q8_0_weight(F, H, seed=701), oracle.q8_0_weight(F, H, seed=702),
+                  oracle.q8_0_weight(H, F, seed=703))
+    gu, _ = Q8Weight.concat(ctx, [Q8Weight.from_gguf(ctx, gb, F, H),
+                                  Q8Weight.from_gguf(ctx, ub, F, H)])
+    y = host(ops.mlp(ctx, gu, Q8Weight.from_gguf(ctx, db, H, F), dev(x), INT8_EXACT))
+    h = oracle.geglu(oracle.matmul(x, gb, F), oracle.matmul(x, ub, F))
+    ref, odd = oracle.matmul(h, db, H), [66, 90, 91]
+    np.testing.assert_array_equal(y[odd], ref[odd])    # a NaN's payload is not defined
+    assert_bits_equal(np.delete(y, odd, 0), np.delete(ref, odd, 0), "geglu epilogue")
