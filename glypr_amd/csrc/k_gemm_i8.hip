@@ -305,7 +305,7 @@ gemm_i8_kernel(const int8_t* __restrict__ A, const float* __restrict__ dA,
 //    issues exactly UPW DMAs per wave (past the last stage it reloads the last
 //    stage into the slot just freed), so "stage s has landed" is the single
 //    constant wait vmcnt((RING-2)*UPW) followed by a barrier;
-//  - stages the per-block scales once, coalesced, in their natural [row][b]
+//  - stages the per-block scales once, coalesced, in [row][b]
 //    layout (dA rows of the tile, then dB rows).
 // LDS layout of a ring slot: A rows then B rows, each [row][128 B] with the
 // 16-byte chunk c of row r stored at chunk c ^ sm_swz(r).  One DMA writes 1 KB
@@ -319,13 +319,21 @@ constexpr int SMALL_NB_MAX = 64;   // K <= 2048
 // measured 2 SQ_LDS_BANK_CONFLICT cycles per read with r & 7 and none with
 // (r >> 1) & 7.
 __device__ __forceinline__ int sm_swz(int r) { return (r >> 1) & 7; }
+// Pitch in floats of the small-M kernels' LDS scale rows.  16 rows' ds_read_b128
+// of one block quad hit 16 different bank quads when the pitch is an odd number
+// of 16-byte chunks; at NB floats they were 16-way conflicts for K = 2048, 8-way
+// for 1024, and the LDS pipe set the time of a stage (100 x 2048 x 512: 8.0 -> 7.2 us,
+// 1000 rows 11.3 -> 10.3, gate/up 333 x 2048 -> 2 x 512 11.7 -> 10.9).  Fewer conflicts
+// (4-way at K = 512) cost less than the wider rows' address arithmetic (gate/up
+// 333 x 512 -> 2 x 2048: 8.8 natural, 9.5 padded), so those keep the natural pitch.
+constexpr int scale_pitch(int nb) { return nb % 32 == 0 ? nb + 4 : nb; }
 
 // WM x WN waves; wave (wm, wn) owns rows 16 wm.. and TNW 16-row B tiles.
 // GEGLU: TNW == 2 (gate tile, up tile of the same 16 h columns) and WN == 2:
 // the 32-wide Q8_0 block of h spans waves wn = 0, 1, which exchange their
 // amax through LDS.  NB = K / 32 blocks, NB % 4 == 0.
 //
-// Scales stay in their natural [row][b] layout in LDS, so the four blocks of
+// Scales stay in [row][b] layout in LDS (see scale_pitch), so the four blocks of
 // a stage are 16 contiguous bytes of a row: per stage a lane reads its four
 // row scales and its TNW column scales with 4 + TNW ds_read_b128.  The stage
 // loop is unrolled by RING so ring slots are compile-time LDS offsets.
@@ -344,7 +352,7 @@ gemm_i8_small_kernel(const int8_t* __restrict__ A, const float* __restrict__ dA,
   constexpr int BN = WN * 16 * TNW;         // B rows per tile
   constexpr int UA = BM / 8, UB = BN / 8;   // 1 KB DMA units per stage
   constexpr int UPW = (UA + UB) / NW;
-  constexpr int SA = NB * BM, SB = NB * BN;
+  constexpr int PB = scale_pitch(NB), SA = PB * BM, SB = PB * BN;
   static_assert(NB % KB == 0 && NB <= SMALL_NB_MAX, "K must be a multiple of 128, <= 2048");
   static_assert((UA + UB) % NW == 0, "stage units must split evenly over the waves");
   static_assert(RING >= 2, "ring needs >= 2 slots");
@@ -374,19 +382,19 @@ gemm_i8_small_kernel(const int8_t* __restrict__ A, const float* __restrict__ dA,
     return (t & 1) ? F + c : c;
   };
 
-  // ---- scales: dA rows [BM][NB] then dB rows [BN][NB], 16 B (four blocks)
+  // ---- scales: dA rows [BM][PB] then dB rows [BN][PB], 16 B (four blocks)
   // per lane; the last unit's spare lanes repeat the last chunk into the slack
-  constexpr int NQ = NB / 4;                    // 16-byte chunks per row
+  constexpr int NQ = NB / 4, PQ = PB / 4;   // 16-byte chunks of a row: filled, in all
   constexpr int SCH = (SA + SB) / 4;            // chunks in all
   for (int c0 = wave * 64; c0 < SCH; c0 += NW * 64) {
     const int c = c0 + lane < SCH ? c0 + lane : SCH - 1;
     const float* src;
     if (c < SA / 4) {
-      const int r = c / NQ, q = c - r * NQ;
+      const int r = c / PQ, q = c - r * PQ < NQ ? c - r * PQ : NQ - 1;
       const int gm = m0 + r < M ? m0 + r : M - 1;
       src = dA + (int64_t)gm * NB + 4 * q;
     } else {
-      const int f = c - SA / 4, r = f / NQ, q = f - r * NQ;
+      const int f = c - SA / 4, r = f / PQ, q = f - r * PQ < NQ ? f - r * PQ : NQ - 1;
       src = dB + (int64_t)b_row(r) * NB + 4 * q;
     }
     dma16_flat(src, lds_u32(sc + 4 * c0));
@@ -426,8 +434,8 @@ gemm_i8_small_kernel(const int8_t* __restrict__ A, const float* __restrict__ dA,
       offB[t][kb] = (BM + brow) * BK + ((ch ^ sm_swz(brow)) << 4) + ((lq & 1) << 3);
     }
   }
-  const float* xrow = sc + (wm * 16 + 4 * lq) * NB;   // row 4 lq + r at xrow + r * NB
-  const float* wrow = sc + SA + (wn * 16 * TNW + l16) * NB;  // tile t at wrow + 16 t NB
+  const float* xrow = sc + (wm * 16 + 4 * lq) * PB;   // row 4 lq + r at xrow + r * PB
+  const float* wrow = sc + SA + (wn * 16 * TNW + l16) * PB;  // tile t at wrow + 16 t PB
   const v4i magic = {MAGIC, MAGIC, MAGIC, MAGIC};
   float acc[TNW][4];
 #pragma unroll
@@ -462,10 +470,10 @@ gemm_i8_small_kernel(const int8_t* __restrict__ A, const float* __restrict__ dA,
         v4f xq[4], wq[TNW];
 #pragma unroll
         for (int rr = 0; rr < 4; rr++)
-          xq[rr] = *reinterpret_cast<const v4f*>(xrow + rr * NB + st * KB);
+          xq[rr] = *reinterpret_cast<const v4f*>(xrow + rr * PB + st * KB);
 #pragma unroll
         for (int t = 0; t < TNW; t++)
-          wq[t] = *reinterpret_cast<const v4f*>(wrow + t * 16 * NB + st * KB);
+          wq[t] = *reinterpret_cast<const v4f*>(wrow + t * 16 * PB + st * KB);
 #pragma unroll
         for (int kb = 0; kb < KB; kb++)
 #pragma unroll
@@ -598,7 +606,7 @@ gemm_i8_geglu8_kernel(const int8_t* __restrict__ A, const float* __restrict__ dA
   constexpr int K = NB * QK, NST = NB / KB;
   constexpr int NW = 4, BM = 16, BN = 64;
   constexpr int UA = BM / 8, UB = BN / 8, UN = UA + UB;   // 2 + 8 DMA units per stage
-  constexpr int SA = NB * BM, SB = NB * BN;
+  constexpr int PB = scale_pitch(NB), SA = PB * BM, SB = PB * BN;
   static_assert(NB % KB == 0 && NB <= SMALL_NB_MAX, "K must be a multiple of 128, <= 2048");
   static_assert(RING >= 2, "ring needs >= 2 slots");
   constexpr int SLOT = (BM + BN) * BK;
@@ -617,17 +625,17 @@ gemm_i8_geglu8_kernel(const int8_t* __restrict__ A, const float* __restrict__ dA
     return (nl & 8) ? F + c : c;
   };
 
-  constexpr int NQ = NB / 4;
+  constexpr int NQ = NB / 4, PQ = PB / 4;   // 16-byte chunks of a row: filled, in all
   constexpr int SCH = (SA + SB) / 4;
   for (int c0 = wave * 64; c0 < SCH; c0 += NW * 64) {
     const int c = c0 + lane < SCH ? c0 + lane : SCH - 1;
     const float* src;
     if (c < SA / 4) {
-      const int r = c / NQ, q = c - r * NQ;
+      const int r = c / PQ, q = c - r * PQ < NQ ? c - r * PQ : NQ - 1;
       const int gm = m0 + r < M ? m0 + r : M - 1;
       src = dA + (int64_t)gm * NB + 4 * q;
     } else {
-      const int f = c - SA / 4, r = f / NQ, q = f - r * NQ;
+      const int f = c - SA / 4, r = f / PQ, q = f - r * PQ < NQ ? f - r * PQ : NQ - 1;
       src = dB + (int64_t)b_row(r) * NB + 4 * q;
     }
     dma16_flat(src, lds_u32(sc + 4 * c0));
@@ -665,8 +673,8 @@ gemm_i8_geglu8_kernel(const int8_t* __restrict__ A, const float* __restrict__ dA
     const int brow = wave * 16 + l16;
     offB[kb] = (BM + brow) * BK + ((ch ^ sm_swz(brow)) << 4) + ((lq & 1) << 3);
   }
-  const float* xrow = sc + (4 * lq) * NB;
-  const float* wrow = sc + SA + (wave * 16 + l16) * NB;
+  const float* xrow = sc + (4 * lq) * PB;
+  const float* wrow = sc + SA + (wave * 16 + l16) * PB;
   const v4i magic = {MAGIC, MAGIC, MAGIC, MAGIC};
   float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 
@@ -694,7 +702,7 @@ gemm_i8_geglu8_kernel(const int8_t* __restrict__ A, const float* __restrict__ dA
         v4f xq[4];
 #pragma unroll
         for (int rr = 0; rr < 4; rr++)
-          xq[rr] = *reinterpret_cast<const v4f*>(xrow + rr * NB + st * KB);
+          xq[rr] = *reinterpret_cast<const v4f*>(xrow + rr * PB + st * KB);
         const v4f wq = *reinterpret_cast<const v4f*>(wrow + st * KB);
 #pragma unroll
         for (int kb = 0; kb < KB; kb++) {
@@ -812,7 +820,7 @@ gemm_i8_pro_kernel(const float* __restrict__ X, const float* __restrict__ nw, fl
   constexpr int BN = WN * 16 * TNW;
   constexpr int UB = BN / 8;               // 1 KB DMA units per stage
   constexpr int UPW = UB / NW;
-  constexpr int SA = NB * BM, SB = NB * BN;
+  constexpr int PB = scale_pitch(NB), SA = PB * BM, SB = PB * BN;
   constexpr int SLOT = BN * BK;
   constexpr int LPR = NW * 64 / BM;        // lanes per row in the prologue
   constexpr int PARTS = LPR / 8;           // 8-lane groups per row
@@ -834,12 +842,12 @@ gemm_i8_pro_kernel(const float* __restrict__ X, const float* __restrict__ nw, fl
   // B row of tile-local row nl (rows past N repeat the last one; never stored)
   auto b_row = [&](int nl) -> int { return n0 + nl < N ? n0 + nl : N - 1; };
 
-  // ---- B scales [BN][NB] by DMA, 16 B (four blocks) per lane
-  constexpr int NQ = NB / 4;
+  // ---- B scales [BN][PB] by DMA, 16 B (four blocks) per lane
+  constexpr int NQ = NB / 4, PQ = PB / 4;   // 16-byte chunks of a row: filled, in all
   constexpr int SCB = SB / 4;
   for (int c0 = wave * 64; c0 < SCB; c0 += NW * 64) {
     const int c = c0 + lane < SCB ? c0 + lane : SCB - 1;
-    const int r = c / NQ, q = c - r * NQ;
+    const int r = c / PQ, q = c - r * PQ < NQ ? c - r * PQ : NQ - 1;
     dma16_flat(dB + (int64_t)b_row(r) * NB + 4 * q, lds_u32(sc + SA + 4 * c0));
   }
   // ---- B stages: this wave's DMA units (8 rows x 128 B each)
@@ -917,7 +925,7 @@ gemm_i8_pro_kernel(const float* __restrict__ X, const float* __restrict__ nw, fl
 #pragma unroll
       for (int i = 1; i < G; i++) asel = pj == i ? am[i] : asel;
       const QScale q = q8_scale(asel);
-      if (pj < G) sc[pr * NB + part * BPP + g0 + pj] = q.dq;
+      if (pj < G) sc[pr * PB + part * BPP + g0 + pj] = q.dq;
 #pragma unroll
       for (int i = 0; i < G; i++) {
         const float id = bcast8(q.id, i);
@@ -945,8 +953,8 @@ gemm_i8_pro_kernel(const float* __restrict__ X, const float* __restrict__ nw, fl
       offB[t][kb] = brow * BK + ((ch ^ sm_swz(brow)) << 4) + ((lq & 1) << 3);
     }
   }
-  const float* xrow = sc + (4 * lq) * NB;                    // row 4 lq + r at xrow + r NB
-  const float* wrow = sc + SA + (wn * 16 * TNW + l16) * NB;  // tile t at wrow + 16 t NB
+  const float* xrow = sc + (4 * lq) * PB;                    // row 4 lq + r at xrow + r PB
+  const float* wrow = sc + SA + (wn * 16 * TNW + l16) * PB;  // tile t at wrow + 16 t PB
   const v4i magic = {MAGIC, MAGIC, MAGIC, MAGIC};
   float acc[TNW][4];
 #pragma unroll
@@ -982,10 +990,10 @@ gemm_i8_pro_kernel(const float* __restrict__ X, const float* __restrict__ nw, fl
         v4f xq[4], wq[TNW];
 #pragma unroll
         for (int rr = 0; rr < 4; rr++)
-          xq[rr] = *reinterpret_cast<const v4f*>(xrow + rr * NB + st * KB);
+          xq[rr] = *reinterpret_cast<const v4f*>(xrow + rr * PB + st * KB);
 #pragma unroll
         for (int t = 0; t < TNW; t++)
-          wq[t] = *reinterpret_cast<const v4f*>(wrow + t * 16 * NB + st * KB);
+          wq[t] = *reinterpret_cast<const v4f*>(wrow + t * 16 * PB + st * KB);
 #pragma unroll
         for (int kb = 0; kb < KB; kb++)
 #pragma unroll
@@ -1415,7 +1423,7 @@ gemm_i8_qkv_kernel(const int8_t* __restrict__ A, const float* __restrict__ dA,
   constexpr int BM = 16, BN = QKV_HD, TNW = 2;
   constexpr int UA = BM / 8, UB = BN / 8;   // 2 and 32 units of 1 KB per stage
   constexpr int UBW = UB / QKV_NW;          // B units per wave
-  constexpr int SA = NB * BM, SB = NB * BN;
+  constexpr int PB = scale_pitch(NB), SA = PB * BM, SB = PB * BN;
   constexpr int SLOT = (BM + BN) * BK;
   static_assert(NB % KB == 0 && NB <= SMALL_NB_MAX, "K must be a multiple of 128, <= 2048");
   static_assert(UB % QKV_NW == 0 && UA <= QKV_NW && BM * QKV_SP * 4 <= SLOT, "layout");
@@ -1435,18 +1443,18 @@ gemm_i8_qkv_kernel(const int8_t* __restrict__ A, const float* __restrict__ dA,
   const int n0 = slot * BN;
   const int M = T;                        // rows with activations
 
-  // ---- scales: dA rows [BM][NB], then dB rows [BN][NB]
-  constexpr int NQ = NB / 4;
+  // ---- scales: dA rows [BM][PB], then dB rows [BN][PB]
+  constexpr int NQ = NB / 4, PQ = PB / 4;   // 16-byte chunks of a row: filled, in all
   constexpr int SCH = (SA + SB) / 4;
   for (int c0 = wave * 64; c0 < SCH; c0 += QKV_NW * 64) {
     const int c = c0 + lane < SCH ? c0 + lane : SCH - 1;
     const float* src;
     if (c < SA / 4) {
-      const int r = c / NQ, q = c - r * NQ;
+      const int r = c / PQ, q = c - r * PQ < NQ ? c - r * PQ : NQ - 1;
       const int gm = m0 + r < M ? m0 + r : M - 1;
       src = dA + (int64_t)gm * NB + 4 * q;
     } else {
-      const int f = c - SA / 4, r = f / NQ, q = f - r * NQ;
+      const int f = c - SA / 4, r = f / PQ, q = f - r * PQ < NQ ? f - r * PQ : NQ - 1;
       src = dB + (int64_t)(n0 + r) * NB + 4 * q;
     }
     dma16_flat(src, lds_u32(sc + 4 * c0));
@@ -1489,8 +1497,8 @@ gemm_i8_qkv_kernel(const int8_t* __restrict__ A, const float* __restrict__ dA,
       offB[t][kb] = (BM + brow) * BK + ((ch ^ sm_swz(brow)) << 4) + ((lq & 1) << 3);
     }
   }
-  const float* xrow = sc + (4 * lq) * NB;
-  const float* wrow = sc + SA + (wn * 16 * TNW + l16) * NB;
+  const float* xrow = sc + (4 * lq) * PB;
+  const float* wrow = sc + SA + (wn * 16 * TNW + l16) * PB;
   const v4i magic = {MAGIC, MAGIC, MAGIC, MAGIC};
   float acc[TNW][4];
 #pragma unroll
@@ -1544,10 +1552,10 @@ gemm_i8_qkv_kernel(const int8_t* __restrict__ A, const float* __restrict__ dA,
         v4f xq[4], wq[TNW];
 #pragma unroll
         for (int rr = 0; rr < 4; rr++)
-          xq[rr] = *reinterpret_cast<const v4f*>(xrow + rr * NB + st * KB);
+          xq[rr] = *reinterpret_cast<const v4f*>(xrow + rr * PB + st * KB);
 #pragma unroll
         for (int t = 0; t < TNW; t++)
-          wq[t] = *reinterpret_cast<const v4f*>(wrow + t * 16 * NB + st * KB);
+          wq[t] = *reinterpret_cast<const v4f*>(wrow + t * 16 * PB + st * KB);
 #pragma unroll
         for (int kb = 0; kb < KB; kb++)
 #pragma unroll

@@ -55,3 +55,27 @@ def test_geglu_tile_epilogue_bit_exact(ctx, oracle, m, H, F, scale):
     ref, odd = oracle.matmul(h, db, H), [66, 90, 91]
     np.testing.assert_array_equal(y[odd], ref[odd])    # a NaN's payload is not defined
     assert_bits_equal(np.delete(y, odd, 0), np.delete(ref, odd, 0), "geglu epilogue")
+
+
+@pytest.mark.parametrize("m,k,n", [(1, 1024, 33), (17, 2048, 64), (333, 2048, 512),
+                                   (1025, 1024, 31)])
+def test_padded_scale_rows_bit_exact(ctx, oracle, m, k, n):
+    """Small-M kernels at K % 1024 == 0, whose LDS scale rows carry one chunk of
+    padding: plain and RMSNorm matmul, and the gate/up tile of an MLP."""
+    say(f"padded scale rows m={m} k={k} n={n}")
+    x = oracle.normal(m * k, seed=800 + m).reshape(m, k)
+    nw = 1 + 0.1 * oracle.normal(k, seed=801)
+    wb = oracle.q8_0_weight(n, k, seed=802)
+    w = Q8Weight.from_gguf(ctx, wb, n, k)
+    assert_bits_equal(host(ops.q8_0_matmul(ctx, w, dev(x), INT8_EXACT)), oracle.matmul(x, wb, n),
+                      "matmul")
+    assert_bits_equal(host(ops.rmsnorm_q8_0_matmul(ctx, w, dev(x), dev(nw), 1e-6, INT8_EXACT)),
+                      oracle.matmul(oracle.rmsnorm(x, nw, 1e-6), wb, n), "rmsnorm matmul")
+    F = 64
+    gb, ub, db = (oracle.q8_0_weight(F, k, seed=803), oracle.q8_0_weight(F, k, seed=804),
+                  oracle.q8_0_weight(k, F, seed=805))
+    gu, _ = Q8Weight.concat(ctx, [Q8Weight.from_gguf(ctx, gb, F, k),
+                                  Q8Weight.from_gguf(ctx, ub, F, k)])
+    y = host(ops.mlp(ctx, gu, Q8Weight.from_gguf(ctx, db, k, F), dev(x), INT8_EXACT))
+    h = oracle.geglu(oracle.matmul(x, gb, F), oracle.matmul(x, ub, F))
+    assert_bits_equal(y, oracle.matmul(h, db, k), "mlp")
