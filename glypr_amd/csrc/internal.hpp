@@ -131,14 +131,15 @@ hipError_t launch_rmsnorm_quant(const float* x, const float* w, float eps, int64
                                 int64_t dim, int8_t* xq, float* dx, hipStream_t s);
 // The token gather x scale (launch_gather's arithmetic) and the first input
 // RMSNorm + Q8_0 (launch_rmsnorm_quant's) in one launch: writes the gathered
-// rows to h and their normalised Q8_0 to xq / dx.  Ids from host memory
+// rows to h and their normalised Q8_0 (plain_q: Q8_0 of the rows themselves,
+// launch_quantize_planar's) to xq / dx.  Ids from host memory
 // (host_ids, at most GATHER_ARG_IDS) or device memory (dev_ids).  Only for
 // gather_norm_ok shapes.
 bool gather_norm_ok(int64_t rows, int64_t dim);
 hipError_t launch_gather_norm(const int8_t* qs, const float* dw, int64_t dim,
                               const uint32_t* host_ids, const uint32_t* dev_ids, int64_t rows,
                               float scale, const float* w, float eps, float* h, int8_t* xq,
-                              float* dx, hipStream_t s);
+                              float* dx, hipStream_t s, bool plain_q = false);
 hipError_t launch_rmsnorm_bf16(const float* x, const float* w, float eps, int64_t rows,
                                int64_t dim, uint16_t* xb, hipStream_t s);
 hipError_t launch_geglu(const float* g, const float* u, float* out, int64_t n, hipStream_t s);
@@ -166,8 +167,9 @@ hipError_t launch_residual_norm(const float* x, const float* w_post, float* h, c
                                 hipStream_t s, const float* scalar = nullptr,
                                 bool plain_q = false, uint16_t* xb = nullptr,
                                 float* yf = nullptr);
-// x = x * mul + 0 (f32), in place
-hipError_t launch_affine(float* x, int64_t n, float mul, hipStream_t s);
+// y = RMSNorm(x * mul + 0) in f32, x and y may be equal
+hipError_t launch_scaled_rmsnorm(const float* x, float mul, const float* w, float eps, float* y,
+                                 int64_t rows, int64_t dim, hipStream_t s);
 // Q8_0 of geglu(g, u): g [rows][dim], u row r at u + r * u_stride
 hipError_t launch_geglu_quant(const float* g, const float* u, int64_t u_stride, int64_t rows,
                               int64_t dim, int8_t* hq, float* dh, hipStream_t s);
@@ -245,6 +247,13 @@ int gemm_i8_route(int64_t M, int64_t Nrows, int64_t K);
 hipError_t launch_gemm_i8(const int8_t* xq, const float* dx, const int8_t* wq, const float* dw,
                           float* y, int64_t M, int64_t N, int64_t K, int64_t ldc,
                           hipStream_t s, bool fma2 = false);
+// Q8_0 of geglu(x W^T, u) (u row r at u + r * ldu): the per-layer-embedding gate
+// in one launch, for gemm_i8_gate_ok shapes
+bool gemm_i8_gate_ok(int64_t M, int64_t P, int64_t K);
+hipError_t launch_gemm_i8_gate(const int8_t* xq, const float* dx, const int8_t* wq,
+                               const float* dw, const float* u, int64_t ldu, int8_t* hq,
+                               float* dh, int64_t M, int64_t P, int64_t K, hipStream_t s,
+                               bool fma2 = false);
 // Gate/up GEMM ([gate; up] rows, 2F x K) with GeGLU + Q8_0 quantization epilogue:
 // hq int8 [M][F], dh f32 [M][F/32].
 hipError_t launch_gemm_i8_geglu(const int8_t* xq, const float* dx, const int8_t* wq,

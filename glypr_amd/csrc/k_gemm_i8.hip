@@ -329,6 +329,8 @@ __device__ __forceinline__ int sm_swz(int r) { return (r >> 1) & 7; }
 constexpr int scale_pitch(int nb) { return nb % 32 == 0 ? nb + 4 : nb; }
 
 // WM x WN waves; wave (wm, wn) owns rows 16 wm.. and TNW 16-row B tiles.
+// GATE: C is not stored; h = geglu(C, U) (U [M][ldu] f32) leaves as Q8_0 with the
+// GEGLU epilogue, the tile's 32 columns being one block.
 // GEGLU: TNW == 2 (gate tile, up tile of the same 16 h columns) and WN == 2:
 // the 32-wide Q8_0 block of h spans waves wn = 0, 1, which exchange their
 // amax through LDS.  NB = K / 32 blocks, NB % 4 == 0.
@@ -340,12 +342,12 @@ constexpr int scale_pitch(int nb) { return nb % 32 == 0 ? nb + 4 : nb; }
 // Argument order: everything the first DMAs need (operands, scales, M, N)
 // comes first, so that it lies within the 14 argument dwords the hardware
 // preloads into SGPRs; the outputs, used at the end, follow.
-template <int WM, int WN, int TNW, bool GEGLU, bool F2, int RING, int NB>
+template <int WM, int WN, int TNW, bool GEGLU, bool F2, int RING, int NB, bool GATE = false>
 __global__ void __launch_bounds__(WM * WN * 64)
 gemm_i8_small_kernel(const int8_t* __restrict__ A, const float* __restrict__ dA,
                      const int8_t* __restrict__ B, const float* __restrict__ dB, int M, int N,
                      int ldc, int F, float* __restrict__ C, int8_t* __restrict__ Hq,
-                     float* __restrict__ dH) {
+                     float* __restrict__ dH, const float* __restrict__ U, int ldu) {
   constexpr int K = NB * QK, NST = NB / KB;
   constexpr int NW = WM * WN;
   constexpr int BM = WM * 16;
@@ -357,10 +359,11 @@ gemm_i8_small_kernel(const int8_t* __restrict__ A, const float* __restrict__ dA,
   static_assert((UA + UB) % NW == 0, "stage units must split evenly over the waves");
   static_assert(RING >= 2, "ring needs >= 2 slots");
   static_assert(!GEGLU || (TNW == 2 && WN == 2), "GeGLU tile: 2 waves x (gate, up)");
+  static_assert(!GATE || (!GEGLU && TNW == 1 && WN == 2), "gate tile: one Q8_0 block of h");
   constexpr int SLOT = (BM + BN) * BK;
   __shared__ __attribute__((aligned(16))) uint8_t ring[RING * SLOT];
   __shared__ __attribute__((aligned(16))) float sc[SA + SB + 256];
-  __shared__ float amax_x[GEGLU ? WN * BM : 1];
+  __shared__ float amax_x[GEGLU || GATE ? WN * BM : 1];
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -382,6 +385,15 @@ gemm_i8_small_kernel(const int8_t* __restrict__ A, const float* __restrict__ dA,
     return (t & 1) ? F + c : c;
   };
 
+  // the up values of a gate tile, loaded in front of every DMA
+  float up[4];
+  if constexpr (GATE) {
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const int row = m0 + wm * 16 + 4 * (lane >> 4) + r;
+      up[r] = U[(int64_t)(row < M ? row : M - 1) * ldu + n0 + wn * 16 + (lane & 15)];
+    }
+  }
   // ---- scales: dA rows [BM][PB] then dB rows [BN][PB], 16 B (four blocks)
   // per lane; the last unit's spare lanes repeat the last chunk into the slack
   constexpr int NQ = NB / 4, PQ = PB / 4;   // 16-byte chunks of a row: filled, in all
@@ -491,7 +503,7 @@ gemm_i8_small_kernel(const int8_t* __restrict__ A, const float* __restrict__ dA,
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 
   const int grow0 = m0 + wm * 16 + 4 * lq;
-  if constexpr (!GEGLU) {
+  if constexpr (!GEGLU && !GATE) {
 #pragma unroll
     for (int t = 0; t < TNW; t++) {
       const int gn = n0 + wn * 16 * TNW + t * 16 + l16;
@@ -505,11 +517,11 @@ gemm_i8_small_kernel(const int8_t* __restrict__ A, const float* __restrict__ dA,
     // barrier, lane l16 = r of each 16-lane group derives the scale of row
     // 4 lq + r and the group broadcasts it.
     const int nbh = F / QK;
-    const int hc = hc0 + wn * 16 + l16;
+    const int hc = (GATE ? n0 : hc0) + wn * 16 + l16;
     float h[4];
 #pragma unroll
     for (int r = 0; r < 4; r++) {
-      h[r] = geglu_scalar(acc[0][r], acc[1][r]);
+      h[r] = geglu_scalar(acc[0][r], GATE ? up[r] : acc[TNW - 1][r]);
       const float v = max16_nonneg(fmaxf(0.0f, fabsf(h[r])));
       if (l16 == 0) amax_x[wn * BM + wm * 16 + 4 * lq + r] = v;
     }
@@ -535,7 +547,7 @@ hipError_t run_small_nb(const int8_t* xq, const float* dx, const int8_t* wq, con
   constexpr int BM = WM * 16, BN = WN * 16 * TNW;
   dim3 grid((unsigned)((Nrows + BN - 1) / BN), (unsigned)((M + BM - 1) / BM));
   gemm_i8_small_kernel<WM, WN, TNW, GEGLU, F2, RING, NB><<<grid, WM * WN * 64, 0, s>>>(
-      xq, dx, wq, dw, (int)M, (int)Nrows, (int)ldc, (int)F, y, hq, dh);
+      xq, dx, wq, dw, (int)M, (int)Nrows, (int)ldc, (int)F, y, hq, dh, nullptr, 0);
   return hipGetLastError();
 }
 
@@ -1896,6 +1908,27 @@ hipError_t gemm_i8_routed(const int8_t* xq, const float* dx, const int8_t* wq, c
 }
 
 template <bool F2>
+hipError_t gate_nb(const int8_t* xq, const float* dx, const int8_t* wq, const float* dw,
+                   const float* u, int64_t ldu, int8_t* hq, float* dh, int64_t M, int64_t P,
+                   int64_t K, hipStream_t s) {
+  const dim3 grid((unsigned)(P / QK), (unsigned)((M + 15) / 16));
+#define GLYPR_GATE_NB(nb)                                                                  \
+  case nb:                                                                                 \
+    gemm_i8_small_kernel<1, 2, 1, false, F2, 3, nb, true><<<grid, 128, 0, s>>>(            \
+        xq, dx, wq, dw, (int)M, (int)P, 0, (int)P, nullptr, hq, dh, u, (int)ldu);          \
+    return hipGetLastError();
+  switch (K / QK) {
+    GLYPR_GATE_NB(8)
+    GLYPR_GATE_NB(16)
+    GLYPR_GATE_NB(24)
+    GLYPR_GATE_NB(32)
+    default:
+      return hipErrorInvalidValue;
+  }
+#undef GLYPR_GATE_NB
+}
+
+template <bool F2>
 hipError_t geglu_i8_routed(const int8_t* xq, const float* dx, const int8_t* wq, const float* dw,
                            int8_t* hq, float* dh, int64_t M, int64_t F, int64_t K,
                            hipStream_t s) {
@@ -1921,6 +1954,28 @@ hipError_t launch_gemm_i8(const int8_t* xq, const float* dx, const int8_t* wq, c
   if (M == 0 || N == 0) return hipSuccess;
   return fma2 ? gemm_i8_routed<true>(xq, dx, wq, dw, y, M, N, K, ldc, s)
               : gemm_i8_routed<false>(xq, dx, wq, dw, y, M, N, K, ldc, s);
+}
+
+// The PLE gate with its GeGLU and Q8_0 epilogue: where the plain product would
+// take gemm_i8_small_kernel, at the widths it is built for, with h in whole
+// Q8_0 blocks.  333 x 512 x 256: 6.3 us of two launches -> 4.8, and a layer's
+// chain has one dependent launch less.  More rows keep the two launches (the product's
+// large tiles hold no 32 columns of a row in 16-row waves).
+bool gemm_i8_gate_ok(int64_t M, int64_t P, int64_t K) {
+  const int64_t nb = K / QK;
+  return gemm_i8_route(M, P, K) == GEMM_ROUTE_SMALL && P % QK == 0 &&
+         (nb == 8 || nb == 16 || nb == 24 || nb == 32) &&
+         !(big_ok(M, P, K) && tiles_beat_small(M, P, K));
+}
+
+hipError_t launch_gemm_i8_gate(const int8_t* xq, const float* dx, const int8_t* wq,
+                               const float* dw, const float* u, int64_t ldu, int8_t* hq,
+                               float* dh, int64_t M, int64_t P, int64_t K, hipStream_t s,
+                               bool fma2) {
+  if (M == 0) return hipSuccess;
+  if (!gemm_i8_gate_ok(M, P, K)) return hipErrorInvalidValue;
+  return fma2 ? gate_nb<true>(xq, dx, wq, dw, u, ldu, hq, dh, M, P, K, s)
+              : gate_nb<false>(xq, dx, wq, dw, u, ldu, hq, dh, M, P, K, s);
 }
 
 // Few rows: the small-M form (16-row blocks); many rows, or a K the small

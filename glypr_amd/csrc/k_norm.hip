@@ -59,7 +59,8 @@ static hipError_t launch_rmsnorm_generic(const float* x, const float* w, float e
 constexpr int NORM_WAVES_MAX = 4;
 inline int norm_waves(int64_t rows) { return rows <= 256 ? 1 : rows <= 512 ? 2 : 4; }
 
-enum NormOut { OUT_F32 = 0, OUT_Q8 = 1, OUT_BF16 = 2 };
+// OUT_F32_PRE: as OUT_F32, of x * pre + 0 (candle's affine(pre, 0) in front)
+enum NormOut { OUT_F32 = 0, OUT_Q8 = 1, OUT_BF16 = 2, OUT_F32_PRE = 3 };
 
 __device__ __forceinline__ uint32_t bf16_rne(float f) {
   uint32_t u = __float_as_uint(f);
@@ -137,7 +138,7 @@ template <int NV, int MODE, bool CHAIN>
 __global__ void __launch_bounds__(64 * NORM_WAVES_MAX)
 rmsnorm_row_kernel(const float* x, const float* __restrict__ w, float eps, int64_t rows, int dim,
                    float* y, int8_t* __restrict__ xq, float* __restrict__ dx,
-                   uint16_t* __restrict__ xb) {
+                   uint16_t* __restrict__ xb, float pre) {
   extern __shared__ float lds_rows[];
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
@@ -154,6 +155,8 @@ rmsnorm_row_kernel(const float* x, const float* __restrict__ w, float eps, int64
     int c4 = lane + 64 * i;
     v[i] = c4 < n4 ? *reinterpret_cast<const v4f*>(xr + 4 * c4) : v4f{0, 0, 0, 0};
     wv[i] = (w && c4 < n4) ? *reinterpret_cast<const v4f*>(w + 4 * c4) : v4f{1, 1, 1, 1};
+    if constexpr (MODE == OUT_F32_PRE)
+      for (int e = 0; e < 4; e++) v[i][e] = v[i][e] * pre + 0.0f;
   }
   float inv;
   if constexpr (CHAIN) {
@@ -198,7 +201,7 @@ rmsnorm_row_kernel(const float* x, const float* __restrict__ w, float eps, int64
   for (int i = 0; i < NV; i++)
 #pragma unroll
     for (int e = 0; e < 4; e++) yv[i][e] = w ? (v[i][e] * inv) * wv[i][e] : v[i][e] * inv;
-  if constexpr (MODE == OUT_F32) {
+  if constexpr (MODE == OUT_F32 || MODE == OUT_F32_PRE) {
 #pragma unroll
     for (int i = 0; i < NV; i++) {
       const int c4 = lane + 64 * i;
@@ -251,7 +254,8 @@ rmsnorm_row_kernel(const float* x, const float* __restrict__ w, float eps, int64
 template <int NV, int MODE>
 __global__ void __launch_bounds__(256)
 rmsnorm_split_kernel(const float* x, const float* __restrict__ w, float eps, int dim, float* y,
-                     int8_t* __restrict__ xq, float* __restrict__ dx, uint16_t* __restrict__ xb) {
+                     int8_t* __restrict__ xq, float* __restrict__ dx, uint16_t* __restrict__ xb,
+                     float pre) {
   __shared__ __attribute__((aligned(16))) float lrow[NV * 256 + 32];
   const int lane = threadIdx.x & 63;
   const int wv = threadIdx.x >> 6;
@@ -259,15 +263,17 @@ rmsnorm_split_kernel(const float* x, const float* __restrict__ w, float eps, int
   const int n4 = dim >> 2;
   const int c4 = lane + 64 * wv;
   const bool ok = c4 < n4;
-  const v4f v = ok ? *reinterpret_cast<const v4f*>(x + row * dim + 4 * c4) : v4f{0, 0, 0, 0};
+  v4f v = ok ? *reinterpret_cast<const v4f*>(x + row * dim + 4 * c4) : v4f{0, 0, 0, 0};
   const v4f ww = (w && ok) ? *reinterpret_cast<const v4f*>(w + 4 * c4) : v4f{1, 1, 1, 1};
+  if constexpr (MODE == OUT_F32_PRE)
+    for (int e = 0; e < 4; e++) v[e] = v[e] * pre + 0.0f;
   if (ok) stage_chains(lrow, chain_stride(dim), c4, v);
   __syncthreads();
   const float inv = chain_row_inv<NV, true>(lrow, dim, lane, eps);
   v4f yv;
 #pragma unroll
   for (int e = 0; e < 4; e++) yv[e] = w ? (v[e] * inv) * ww[e] : v[e] * inv;
-  if constexpr (MODE == OUT_F32) {
+  if constexpr (MODE == OUT_F32 || MODE == OUT_F32_PRE) {
     if (ok) *reinterpret_cast<v4f*>(y + row * dim + 4 * c4) = yv;
   } else if constexpr (MODE == OUT_BF16) {
     if (ok) {
@@ -298,14 +304,15 @@ inline bool norm_split(int64_t rows, int64_t dim) {
 
 template <int MODE>
 static hipError_t launch_norm(const float* x, const float* w, float eps, int64_t rows, int64_t dim,
-                              float* y, int8_t* xq, float* dx, uint16_t* xb, hipStream_t s) {
+                              float* y, int8_t* xq, float* dx, uint16_t* xb, hipStream_t s,
+                              float pre = 1.0f) {
   if (rows == 0) return hipSuccess;
   if (norm_split(rows, dim)) {
     switch ((dim + 255) / 256) {
 #define NORM_SPLIT_CASE(N)                                                                    \
   case N:                                                                                     \
     rmsnorm_split_kernel<N, MODE><<<(unsigned)rows, 64 * N, 0, s>>>(x, w, eps, (int)dim, y,   \
-                                                                     xq, dx, xb);             \
+                                                                     xq, dx, xb, pre);        \
     break;
       NORM_SPLIT_CASE(1)
       NORM_SPLIT_CASE(2)
@@ -327,10 +334,10 @@ static hipError_t launch_norm(const float* x, const float* w, float eps, int64_t
   case N:                                                                                     \
     if (chain)                                                                                \
       rmsnorm_row_kernel<NK, MODE, true><<<grid, 64 * nw, lds, s>>>(                          \
-          x, w, eps, rows, (int)dim, y, xq, dx, xb);                                          \
+          x, w, eps, rows, (int)dim, y, xq, dx, xb, pre);                                     \
     else                                                                                      \
       rmsnorm_row_kernel<NK, MODE, false><<<grid, 64 * nw, lds, s>>>(                         \
-          x, w, eps, rows, (int)dim, y, xq, dx, xb);                                          \
+          x, w, eps, rows, (int)dim, y, xq, dx, xb, pre);                                     \
     break;
     NORM_CASE(1, 1)
     NORM_CASE(2, 2)
@@ -370,7 +377,10 @@ hipError_t launch_rmsnorm_bf16(const float* x, const float* w, float eps, int64_
 // gather_rows_kernel's arithmetic ((float)q * d, then * scale + 0), writes it
 // to h and stages it for the reference-order chains; the rest is
 // rmsnorm_split_kernel<NV, OUT_Q8>.  Bit-identical to the two launches.
-template <int NV, class Ids>
+// PLAIN: Q8_0 of the gathered row itself (the per-layer projection's operand,
+// gather_rows_kernel + quantize_planar_kernel in one launch: 333 rows of 512
+// 6.4 -> 3.0 us).
+template <int NV, class Ids, bool PLAIN>
 __global__ void __launch_bounds__(256)
 gather_norm_split_kernel(const int8_t* __restrict__ qs, const float* __restrict__ dw, Ids ids,
                          float scale, const float* __restrict__ w, float eps, int dim,
@@ -392,19 +402,18 @@ gather_norm_split_kernel(const int8_t* __restrict__ qs, const float* __restrict_
     const float y = (float)(int8_t)((q >> (8 * e)) & 0xFF) * d;
     v[e] = y * scale + 0.0f;
   }
-  if (ok) {
-    *reinterpret_cast<v4f*>(h + row * dim + 4 * c4) = v;
-    stage_chains(lrow, chain_stride(dim), c4, v);
+  if (ok) *reinterpret_cast<v4f*>(h + row * dim + 4 * c4) = v;
+  v4f yv = v;
+  if constexpr (!PLAIN) {
+    if (ok) stage_chains(lrow, chain_stride(dim), c4, v);
+    __syncthreads();
+    const float inv = chain_row_inv<NV, true>(lrow, dim, lane, eps);
+#pragma unroll
+    for (int e = 0; e < 4; e++) yv[e] = w ? (v[e] * inv) * ww[e] : v[e] * inv;
   }
-  __syncthreads();
-  const float inv = chain_row_inv<NV, true>(lrow, dim, lane, eps);
-  v4f yv;
   float a = 0.0f;
 #pragma unroll
-  for (int e = 0; e < 4; e++) {
-    yv[e] = w ? (v[e] * inv) * ww[e] : v[e] * inv;
-    a = fmaxf(a, fabsf(yv[e]));
-  }
+  for (int e = 0; e < 4; e++) a = fmaxf(a, fabsf(yv[e]));
   const QScale sc = q8_scale(max8(a));
   uint32_t packed = 0;
 #pragma unroll
@@ -421,27 +430,29 @@ bool gather_norm_ok(int64_t rows, int64_t dim) { return rows > 0 && norm_split(r
 hipError_t launch_gather_norm(const int8_t* qs, const float* dw, int64_t dim,
                               const uint32_t* host_ids, const uint32_t* dev_ids, int64_t rows,
                               float scale, const float* w, float eps, float* h, int8_t* xq,
-                              float* dx, hipStream_t s) {
+                              float* dx, hipStream_t s, bool plain_q) {
   if (!gather_norm_ok(rows, dim) || (host_ids && rows > GATHER_ARG_IDS) ||
       (!host_ids && !dev_ids))
     return hipErrorInvalidValue;
   GatherIds arg;
   if (host_ids) memcpy(arg.v, host_ids, (size_t)rows * 4);
   switch ((dim + 255) / 256) {
+#define GATHER_NORM(N, IDS, ids, PLAIN)                                                        \
+  gather_norm_split_kernel<N, IDS, PLAIN><<<(unsigned)rows, 64 * N, 0, s>>>(                   \
+      qs, dw, ids, scale, w, eps, (int)dim, h, xq, dx)
 #define GATHER_NORM_CASE(N)                                                                    \
   case N:                                                                                      \
-    if (host_ids)                                                                              \
-      gather_norm_split_kernel<N, GatherIds><<<(unsigned)rows, 64 * N, 0, s>>>(                \
-          qs, dw, arg, scale, w, eps, (int)dim, h, xq, dx);                                    \
-    else                                                                                       \
-      gather_norm_split_kernel<N, const uint32_t*><<<(unsigned)rows, 64 * N, 0, s>>>(          \
-          qs, dw, dev_ids, scale, w, eps, (int)dim, h, xq, dx);                                \
+    if (host_ids && plain_q) GATHER_NORM(N, GatherIds, arg, true);                             \
+    else if (host_ids) GATHER_NORM(N, GatherIds, arg, false);                                  \
+    else if (plain_q) GATHER_NORM(N, const uint32_t*, dev_ids, true);                          \
+    else GATHER_NORM(N, const uint32_t*, dev_ids, false);                                      \
     break;
     GATHER_NORM_CASE(1)
     GATHER_NORM_CASE(2)
     GATHER_NORM_CASE(3)
     GATHER_NORM_CASE(4)
 #undef GATHER_NORM_CASE
+#undef GATHER_NORM
     default:
       return hipErrorInvalidValue;
   }
@@ -740,18 +751,27 @@ hipError_t launch_geglu(const float* g, const float* u, float* out, int64_t n, h
 // candle's Tensor * f64 on f32 (affine(mul, 0)): y = v * f32(mul) + 0.0f, two
 // roundings (the + 0 turns a -0 product into +0).
 // ---------------------------------------------------------------------------
-__global__ void __launch_bounds__(256) affine_kernel(float* x, int64_t n, float mul) {
+__global__ void __launch_bounds__(256) affine_kernel(const float* x, float* y, int64_t n,
+                                                     float mul) {
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
        i += (int64_t)gridDim.x * blockDim.x)
-    x[i] = x[i] * mul + 0.0f;
+    y[i] = x[i] * mul + 0.0f;
 }
 
-hipError_t launch_affine(float* x, int64_t n, float mul, hipStream_t s) {
+// RMSNorm(x * mul + 0): one pass over x where the row kernels take the width
+// (666 rows of 256: 4.6 us of two launches -> 2.7), else the scale as a launch of
+// its own before the generic kernel.
+hipError_t launch_scaled_rmsnorm(const float* x, float mul, const float* w, float eps, float* y,
+                                 int64_t rows, int64_t dim, hipStream_t s) {
+  if (dim % 4 == 0 && dim <= 2048)
+    return launch_norm<OUT_F32_PRE>(x, w, eps, rows, dim, y, nullptr, nullptr, nullptr, s, mul);
+  const int64_t n = rows * dim;
   if (n == 0) return hipSuccess;
   int64_t grid = (n + 255) / 256;
   if (grid > 65536) grid = 65536;
-  affine_kernel<<<(unsigned)grid, 256, 0, s>>>(x, n, mul);
-  return hipGetLastError();
+  affine_kernel<<<(unsigned)grid, 256, 0, s>>>(x, y, n, mul);
+  const hipError_t e = hipGetLastError();
+  return e != hipSuccess ? e : launch_rmsnorm_generic(y, w, eps, y, rows, dim, s);
 }
 
 // ---------------------------------------------------------------------------

@@ -457,14 +457,16 @@ int forward_rows(glypr_model* m, glypr_hip_ctx* ctx, const Rows& rows, float* hi
   // model.rs:507-508: Embedding::forward, then * embed_scale (f64 sqrt(hidden) as f32)
   const float embed_scale = (float)sqrt((double)H);
   const int64_t P = c.ple_dim, NL = c.n_layers;
-  // Without PLE the gather and layer 0's input norm run as one launch (the
-  // PLE projection would need xq for its own operand in between).
+  // Without PLE the gather and layer 0's input norm run as one launch; with it
+  // the gather and the Q8_0 of h that the per-layer projection takes.
+  const bool gather_q8 = P > 0 && gather_norm_ok(t, H);
   const bool gather_norm = P == 0 && !m->dense && gather_norm_ok(t, H);
-  if (gather_norm)
+  if (gather_norm || gather_q8)
     LAUNCH(GLYPR_K_GATHER, s,
            launch_gather_norm(m->token_embd.w->qs(), m->token_embd.w->dw(), H, rows.host_ids,
                               rows.host_ids ? nullptr : m->ids.as<uint32_t>(), t, embed_scale,
-                              m->layers[0].input_layernorm.weight, c.eps, h, xq, dx, s),
+                              gather_q8 ? nullptr : m->layers[0].input_layernorm.weight, c.eps, h,
+                              xq, dx, s, gather_q8),
            "gather + input norm launch");
   else if (rows.host_ids)
     LAUNCH(GLYPR_K_GATHER, s,
@@ -481,14 +483,15 @@ int forward_rows(glypr_model* m, glypr_hip_ctx* ctx, const Rows& rows, float* hi
   // affine), RMSNorm over ple_dim.  Layer l's input is row t*NL + l of [t*NL][P].
   float* ple = dev_f32(m->ple);
   if (P > 0) {
-    LAUNCH(GLYPR_K_QUANTIZE, s, launch_quantize_planar(h, t, H, xq, dx, s), "quantize launch");
+    if (!gather_q8)
+      LAUNCH(GLYPR_K_QUANTIZE, s, launch_quantize_planar(h, t, H, xq, dx, s), "quantize launch");
     const glypr_q8w* wpl = m->ple_projection.w;
     LAUNCH(GLYPR_K_GEMM_I8, s,
            launch_gemm_i8(xq, dx, wpl->qs(), wpl->dw(), ple, t, NL * P, H, NL * P, s, m->fma2),
            "per-layer projection launch");
-    LAUNCH(GLYPR_K_RMSNORM, s, launch_affine(ple, t * NL * P, (float)pow((double)H, -0.5), s),
-           "per-layer scale launch");
-    LAUNCH(GLYPR_K_RMSNORM, s, launch_rmsnorm(ple, m->ple_norm.weight, c.eps, ple, t * NL, P, s),
+    LAUNCH(GLYPR_K_RMSNORM, s,
+           launch_scaled_rmsnorm(ple, (float)pow((double)H, -0.5), m->ple_norm.weight, c.eps, ple,
+                                 t * NL, P, s),
            "per-layer norm launch");
   }
   if (m->dense) return forward_dense(m, ctx, rows, hidden, tokens_out, s);
@@ -582,13 +585,21 @@ int forward_rows(glypr_model* m, glypr_hip_ctx* ctx, const Rows& rows, float* hi
            "residual_norm launch");
     // ---- TextPLEBlock::forward_with_scalar (ple.rs:118-145)
     const glypr_q8w* wg = L.ple_block.gate.w;
-    LAUNCH(GLYPR_K_GEMM_I8, s,
-           launch_gemm_i8(xq, dx, wg->qs(), wg->dw(), dev_f32(m->ple_gate), t, P, H, P, s, m->fma2),
-           "per-layer gate launch");
-    LAUNCH(GLYPR_K_GEGLU, s,
-           launch_geglu_quant(dev_f32(m->ple_gate), ple + (int64_t)li * P, NL * P, t, P,
-                              m->hq.as<int8_t>(), dev_f32(m->dh), s),
-           "per-layer geglu launch");
+    if (gemm_i8_gate_ok(t, P, H)) {
+      LAUNCH(GLYPR_K_GEMM_I8_GEGLU, s,
+             launch_gemm_i8_gate(xq, dx, wg->qs(), wg->dw(), ple + (int64_t)li * P, NL * P,
+                                 m->hq.as<int8_t>(), dev_f32(m->dh), t, P, H, s, m->fma2),
+             "per-layer gate launch");
+    } else {
+      LAUNCH(GLYPR_K_GEMM_I8, s,
+             launch_gemm_i8(xq, dx, wg->qs(), wg->dw(), dev_f32(m->ple_gate), t, P, H, P, s,
+                            m->fma2),
+             "per-layer gate launch");
+      LAUNCH(GLYPR_K_GEGLU, s,
+             launch_geglu_quant(dev_f32(m->ple_gate), ple + (int64_t)li * P, NL * P, t, P,
+                                m->hq.as<int8_t>(), dev_f32(m->dh), s),
+             "per-layer geglu launch");
+    }
     const glypr_q8w* wpj = L.ple_block.projection.w;
     LAUNCH(GLYPR_K_GEMM_I8, s,
            launch_gemm_i8(m->hq.as<int8_t>(), dev_f32(m->dh), wpj->qs(), wpj->dw(),
