@@ -32,12 +32,13 @@ double plan_parts(AttnPlan& p, int64_t blocks, int64_t nkb, double start, double
   int64_t most = nkb < ATTN_MAX_PARTS ? nkb : ATTN_MAX_PARTS;
   if (blocks >= ATTN_BLOCKS) most = 1;
   for (int64_t want = 1; want <= most; want++) {
+    const double split = want > 1 ? 3.0 + want * part_bytes * 2 / 5.5e6 : 0.0;
+    if (want > 1 && start + split >= best) break;   // so do all that follow
     const int64_t per = (nkb + want - 1) / want;
     if ((nkb + per - 1) / per != want) continue;
     const int64_t rounds = (blocks * want + ATTN_BLOCKS - 1) / ATTN_BLOCKS;
     const bool full = blocks * want * 5 > ATTN_BLOCKS * 3;
-    const double c = rounds * (start + per * (full ? tile_full : tile)) +
-                     (want > 1 ? 3.0 + want * part_bytes * 2 / 5.5e6 : 0.0);
+    const double c = rounds * (start + per * (full ? tile_full : tile)) + split;
     if (want == 1 || c < best) {
       best = c;
       p.per = (int)per;
@@ -96,8 +97,9 @@ bool attention_supported(int64_t T, int64_t nq, int64_t nkv, int64_t hd, int64_t
     return false;
   if (T <= 0) return true;
   if (!attention_rows_ok(T, hd)) return false;
-  // the combine holds one partition per lane
-  return attn_plan(T, attn_padded_len(T), hd, nq, nkv, window, false).kparts <= 64;
+  // A block's keys: at most 64 partitions (the combine holds one per lane) of 64
+  // key tiles, 131,072 keys
+  return key_tiles(T, window, hd == 512 ? 16 : 64) <= ATTN_MAX_PARTS * 64;
 }
 
 size_t attention_scratch_floats(int64_t T, int64_t nq, int64_t nkv, int64_t hd, int64_t window,
