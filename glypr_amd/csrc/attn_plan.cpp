@@ -105,9 +105,9 @@ bool attention_supported(int64_t T, int64_t nq, int64_t nkv, int64_t hd, int64_t
 size_t attention_scratch_floats(int64_t T, int64_t nq, int64_t nkv, int64_t hd, int64_t window,
                                 int64_t rows) {
   const int64_t tp = rows > 0 ? rows : attn_padded_len(T);
-  int kp = 1;
-  for (const bool segments : {false, true}) {
-    const int k = attn_plan(T, tp, hd, nq, nkv, window, segments).kparts;
+  int kp = attn_plan(T, tp, hd, nq, nkv, window, false).kparts;
+  if (nq / nkv % 2 != 0) {   // segments change the plan of 1 and 3 heads only
+    const int k = attn_plan(T, tp, hd, nq, nkv, window, true).kparts;
     kp = k > kp ? k : kp;
   }
   return (size_t)(kp * tp * nq * (hd + 2));
@@ -131,7 +131,8 @@ size_t attention_scratch_bound(int64_t max_t, int64_t cap_rows, int64_t nq, int6
         break;
       }
     }
-    if (tk == max_t) break;
+    // (past the widest band every tk plans alike, over fewer row counts)
+    if (tk == max_t || (window > 0 && key_tiles(tk, window, 128) * ATTN_AK < tk)) break;
   }
   return best;
 }
