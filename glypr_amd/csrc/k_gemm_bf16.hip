@@ -237,6 +237,16 @@ hipError_t run(const uint16_t* xb, const int8_t* wq, const float* dw, float* y, 
 // (dequant16: the exact q*d, then bf16 round-to-nearest-even, as the staged
 // path) and runs two MFMA k-steps on K {0..7, 16..23} and {8..15, 24..31} of
 // the block; A and B use the same order, so every product is formed once.
+// AHEAD: a stage's two blocks are dequantized in front of its products, and every
+// k-step takes the TM tiles in turn: no product waits on the one right before it,
+// and the A fragments of the second block load under the first's.  For 128-row tiles
+// with at most two workgroups on a CU (6000 x 768 x 768 24.8 -> 23.0 us, 2100 x 768 x 2304
+// 20.6 -> 19.4, 8190 x 1152 x 768 34.3 -> 32.9); three hide each other's latency (16384 x
+// 768 x 1280 57.5 both ways, 12000 x 768 x 1000 41.0 -> 41.5), and lower tiles are 1 to 3 %
+// slower for it (300 x 1024 x 512 12.2 -> 12.5).
+// Bound: latency at three waves per SIMD.  Wider waves (128 x 64: half the LDS
+// reads per product, two per SIMD) were slower: 8190 x 768 x 1280 35.7 -> 39.0 us in
+// 128 x 256 tiles, 37.8 in 128 x 128 tiles of two waves.
 // XCD-aware tile order as in the int8 large-M kernel; at TM = 4 50 KB of LDS and
 // ~120 VGPRs, so three workgroups share a CU.  The 128-column tile (rather than
 // 256) keeps the grids of the C3 projections near whole rounds of 768
@@ -249,7 +259,7 @@ hipError_t run(const uint16_t* xb, const int8_t* wq, const float* dw, float* y, 
 constexpr int BFB_BN = 128, BFB_BK = 64;
 
 // TM 32-row MFMA tiles per wave (BM = 32 TM rows per workgroup).
-template <bool GEGLU, int TM>
+template <bool GEGLU, int TM, bool AHEAD>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3)))
 gemm_bf16_big_kernel(const uint16_t* __restrict__ A, const int8_t* __restrict__ B,
                      const float* __restrict__ dB, float* __restrict__ C,
@@ -354,6 +364,19 @@ gemm_bf16_big_kernel(const uint16_t* __restrict__ A, const int8_t* __restrict__ 
     __syncthreads();
     if (st + 1 < nst) issue(st + 1, r ^ 1);
     const uint8_t* slot = ring + r * SLOT;
+    v8bf b[2][2];   // [block][k-step]
+    auto dequant = [&](int p) {
+      const v4i q = *reinterpret_cast<const v4i*>(slot + offB[p]);
+      const float d = *reinterpret_cast<const float*>(slot + offS[p]);
+      v4i lo, hi;
+      dequant16(q, d, lo, hi);
+      b[p][0] = __builtin_bit_cast(v8bf, lo);
+      b[p][1] = __builtin_bit_cast(v8bf, hi);
+    };
+    if constexpr (AHEAD) {
+      dequant(0);
+      dequant(1);
+    }
 #pragma unroll
     for (int p = 0; p < 2; p++) {
       v8bf a[TM][2];
@@ -362,15 +385,11 @@ gemm_bf16_big_kernel(const uint16_t* __restrict__ A, const int8_t* __restrict__ 
 #pragma unroll
         for (int h = 0; h < 2; h++)
           a[tm][h] = *reinterpret_cast<const v8bf*>(slot + offA[tm][p][h]);
-      const v4i q = *reinterpret_cast<const v4i*>(slot + offB[p]);
-      const float d = *reinterpret_cast<const float*>(slot + offS[p]);
-      v4i lo, hi;
-      dequant16(q, d, lo, hi);
-      const v8bf b0 = __builtin_bit_cast(v8bf, lo), b1 = __builtin_bit_cast(v8bf, hi);
+      if constexpr (!AHEAD) dequant(p);
 #pragma unroll
-      for (int tm = 0; tm < TM; tm++) {
-        acc[tm] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[tm][0], b0, acc[tm], 0, 0, 0);
-        acc[tm] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[tm][1], b1, acc[tm], 0, 0, 0);
+      for (int i = 0; i < 2 * TM; i++) {
+        const int tm = AHEAD ? i % TM : i >> 1, h = AHEAD ? i / TM : i & 1;
+        acc[tm] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[tm][h], b[p][h], acc[tm], 0, 0, 0);
       }
     }
   }
@@ -435,13 +454,13 @@ gemm_bf16_big_kernel(const uint16_t* __restrict__ A, const int8_t* __restrict__ 
   }
 }
 
-template <bool GEGLU, int TM>
+template <bool GEGLU, int TM, bool AHEAD = false>
 hipError_t run_big(const uint16_t* xb, const int8_t* wq, const float* dw, float* y, uint16_t* hb,
                    int64_t M, int64_t Nrows, int64_t K, int64_t ldc, int64_t F, hipStream_t s) {
   constexpr int BM = 32 * TM;
   const int64_t tiles_n = (Nrows + BFB_BN - 1) / BFB_BN;
   const int64_t tiles = ((M + BM - 1) / BM) * tiles_n;
-  gemm_bf16_big_kernel<GEGLU, TM><<<dim3((unsigned)tiles), 256, 0, s>>>(
+  gemm_bf16_big_kernel<GEGLU, TM, AHEAD><<<dim3((unsigned)tiles), 256, 0, s>>>(
       xb, wq, dw, y, hb, (int)M, (int)Nrows, (int)K, (int)ldc, (int)F, (int)tiles_n);
   return hipGetLastError();
 }
@@ -461,6 +480,8 @@ hipError_t run_big_rows(const uint16_t* xb, const int8_t* wq, const float* dw, f
     return run_big<GEGLU, 1>(xb, wq, dw, y, hb, M, Nrows, K, ldc, F, s);
   if (M <= 2048 || (M + 63) / 64 * tiles_n <= 384)
     return run_big<GEGLU, 2>(xb, wq, dw, y, hb, M, Nrows, K, ldc, F, s);
+  if ((M + 127) / 128 * tiles_n <= 512)
+    return run_big<GEGLU, 4, true>(xb, wq, dw, y, hb, M, Nrows, K, ldc, F, s);
   return run_big<GEGLU, 4>(xb, wq, dw, y, hb, M, Nrows, K, ldc, F, s);
 }
 
