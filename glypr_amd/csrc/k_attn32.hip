@@ -130,11 +130,13 @@ attn_tile32_kernel(const f16* __restrict__ q16, const f16* __restrict__ kk,
   const int vl = (lane >> 2) * Tp * 2 + (((lane & 3) ^ ((lane >> 4) & 3)) << 4);
   auto issue_k = [&](int kb, int sl) {
     const int8_t* base = reinterpret_cast<const int8_t*>(kbase + (int64_t)kb * TILE_H);
+    int kl_ = kl;   // opaque with two waves: sixteen offsets held across the loop would spill
+    if constexpr (NWV == 2) asm volatile("" : "+v"(kl_));
 #pragma unroll
     for (int j = 0; j < (KU + NWV - 1) / NWV; j++) {
       const int u = w + NWV * j;
       if (KU % NWV == 0 || u < KU)
-        dma16(base + u * 1024, kl ^ ((key_of_row(u * KRPU) & 15) << 4),
+        dma16(base + u * 1024, kl_ ^ ((key_of_row(u * KRPU) & 15) << 4),
               lds_u32(&Ks[sl][u * 512]));
     }
   };
@@ -164,7 +166,9 @@ attn_tile32_kernel(const f16* __restrict__ q16, const f16* __restrict__ kk,
   const int vfo = l31 * A32_K;
   const int vx = (l31 >> 2) & 3;
 
-  float m_run = -INFINITY, l_run = 0.0f, thr = -INFINITY, mlog = 0.0f;
+  // l_run + l_lo: the sum of the tiles' sums with the additions' rounding errors
+  // kept apart, so a partition of any length is as exact as one of few tiles
+  float m_run = -INFINITY, l_run = 0.0f, l_lo = 0.0f, thr = -INFINITY, m_use = 0.0f;
   v16f o[NT];
 #pragma unroll
   for (int t = 0; t < NT; t++)
@@ -208,10 +212,11 @@ attn_tile32_kernel(const f16* __restrict__ q16, const f16* __restrict__ kk,
     if (__any(mloc > thr)) {
       const float mx = pair_max32(mloc);
       const float m_new = mx > thr ? mx : m_run;
-      const float m_use = m_new == -INFINITY ? 0.0f : m_new;
+      m_use = m_new == -INFINITY ? 0.0f : m_new;
       if (__any(m_run != -INFINITY)) {   // O and l are still zero otherwise
         const float alpha = __expf(m_run - m_use);
         l_run *= alpha;
+        l_lo *= alpha;
         acc_settle<HD>(o);
 #pragma unroll
         for (int t = 0; t < NT; t++) {
@@ -222,7 +227,6 @@ attn_tile32_kernel(const f16* __restrict__ q16, const f16* __restrict__ kk,
       }
       m_run = m_new;
       thr = m_new + ATTN_TAU;
-      mlog = m_use * ATTN_LOG2E;
     }
     // K of tile kb+1 and V^T of tile kb have landed, for every wave
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -246,6 +250,7 @@ attn_tile32_kernel(const f16* __restrict__ q16, const f16* __restrict__ kk,
     // exponentials of tile kb, then O^T += V^T P^T; fragments one chunk ahead
     constexpr int CH = HD == 512 ? 4 : 4;
     v8h fr[2][CH];
+    float ps[2] = {0.0f, 0.0f};
 #pragma unroll
     for (int e = 0; e < CH; e++) fr[0][e] = kfrag(e);
 #pragma unroll
@@ -260,11 +265,19 @@ attn_tile32_kernel(const f16* __restrict__ q16, const f16* __restrict__ kk,
 #pragma unroll
       for (int e = 0; e < EPC; e++) {
         const int r = c * EPC + e;
-        const float pv = __builtin_amdgcn_exp2f(fmaf(sc[r], ATTN_LOG2E, -mlog));
-        l_run += pv;
+        // (the difference first: a product m * log2(e) rounded on its own would
+        // shift partitions and rescales against each other by |m| 2^-24; one
+        // instruction more each, T = 8192 at head_dim 512: 588 -> 593 us)
+        const float pv = __expf(sc[r] - m_use);
+        ps[r >> 3] += pv;
         pf[r >> 3][r & 7] = (f16)pv;
       }
       __builtin_amdgcn_sched_barrier(0);
+    }
+    {
+      const float pt = ps[0] + ps[1], l_new = l_run + pt;
+      l_lo += pt - (l_new - l_run);
+      l_run = l_new;
     }
     constexpr int PB = (NS / CH) & 1;     // the buffer the first V^T chunk is in
 #pragma unroll
@@ -282,7 +295,7 @@ attn_tile32_kernel(const f16* __restrict__ q16, const f16* __restrict__ kk,
     sc = sn;
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  l_run = pair_sum32(l_run);
+  l_run = pair_sum32(l_run + l_lo);
   acc_settle<HD>(o);
 
   if (c0 + w >= c1) return;   // a spare wave (no barrier follows)
