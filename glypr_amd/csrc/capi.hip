@@ -842,6 +842,12 @@ int glypr_internal_gemm_i8_route(int64_t m, int64_t n, int64_t k, int prologue) 
   return gemm_i8_route(m, n, k);
 }
 
+// Likewise the dense bf16 GEMM's tile: rows << 16 | columns.
+int glypr_internal_dense_tile(int64_t m, int64_t n) {
+  const DenseTile t = dense_tile(m, n);
+  return t.rows << 16 | t.cols;
+}
+
 static const char* const kKernelNames[GLYPR_K_COUNT] = {
     "quantize",   "rmsnorm_quant",  "gemm_i8", "gemm_i8_geglu", "to_bf16", "rmsnorm_bf16",
     "gemm_bf16",  "gemm_bf16_geglu", "rmsnorm", "geglu",         "gather",  "dequant",

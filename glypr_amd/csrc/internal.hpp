@@ -287,6 +287,11 @@ hipError_t launch_gemm_i8_pro(const float* x, const float* nw, float eps, bool n
 // y = xb . wb^T (xb bf16 [M][K], wb bf16 [N][K]), f32 out; the GeGLU form takes
 // wb = [gate; up] (2F rows) and writes h bf16 [M][F].  K % 64 == 0.
 bool gemm_bf16w_ok(int64_t M, int64_t Nrows, int64_t K);
+// The tile of launch_gemm_bf16w's grid
+struct DenseTile {
+  int rows, cols;
+};
+DenseTile dense_tile(int64_t M, int64_t N);
 hipError_t launch_gemm_bf16w(const uint16_t* xb, const uint16_t* wb, float* y, int64_t M,
                              int64_t N, int64_t K, int64_t ldc, hipStream_t s);
 hipError_t launch_gemm_bf16w_geglu(const uint16_t* xb, const uint16_t* wb, uint16_t* hb,

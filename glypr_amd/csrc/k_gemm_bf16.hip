@@ -853,21 +853,37 @@ hipError_t run_dense_tile(const uint16_t* xb, const uint16_t* wb, float* y, uint
   return hipGetLastError();
 }
 
+}  // namespace
+
 // The plain GEMM's tile.  Up to 640 tiles of 64 x 64 (2.5 per CU) the 128 x 128
 // grid leaves most CUs idle and each workgroup alone with its DMA latency:
 // 64 x 64 tiles on a three-slot ring (300 x 1152 x 768: 13.7 -> 6.7 us; 1000 x
-// 2048 x 512: 21.0 -> 9.6; 3001 x 1152 x 768: 15.6 -> 13.5).  Above, 64 x 128
-// tiles (three workgroups per CU) where 128 x 128 ones fill at most one per CU
-// or N is below 2048 (8192 x 768 x 1280: 29.5 -> 27.0; 16384: 54.4 -> 48.7);
-// 5000 x 768 x 2304 stays at 128 x 128 (29.5 against 32.7), which reads a third
-// less LDS per product.
+// 2048 x 512: 21.0 -> 9.6; 3001 x 1152 x 768: 15.6 -> 13.5).  Above, a 128 x 128
+// tile reads a third less LDS per product than two of 64 x 128, so the lower one
+// pays only where its grid rounds up to less work per CU: fewer than twice the
+// tiles (128 x 128 -> 64 x 128, calls with the conversion: 8190 x 768 x 1280, 3 and
+// 5 per CU, 36.4 -> 34.3 us; 12000 x 768 x 768, 3 and 5, 36.9 -> 33.9; at twice the
+// tiles 6000 x 768 x 1280 27.4 -> 28.0, 10000 x 1152 x 768 36.3 -> 40.6, 16384 x 2048
+// x 512 67.3 -> 77.4), and below a tile per CU.  From 2048 columns on the grid
+// is long enough for 128 x 128 (5000 x 768 x 2304 34.4 against 37.6).
+DenseTile dense_tile(int64_t M, int64_t N) {
+  auto tiles = [&](int64_t bm, int64_t bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
+  if (tiles(64, 64) <= 640) return {64, 64};
+  const int64_t high = tiles(128, 128), low = tiles(64, 128);
+  if (high <= 256 || (N < 2048 && (low + 255) / 256 < 2 * ((high + 255) / 256))) return {64, 128};
+  return {128, 128};
+}
+
+namespace {
+
 template <bool GEGLU>
 hipError_t run_dense(const uint16_t* xb, const uint16_t* wb, float* y, uint16_t* hb, int64_t M,
                      int64_t Nrows, int64_t K, int64_t ldc, int64_t F, hipStream_t s) {
   if constexpr (!GEGLU) {
-    if (((M + 63) / 64) * ((Nrows + 63) / 64) <= 640)
+    const DenseTile t = dense_tile(M, Nrows);
+    if (t.cols == 64)
       return run_dense_tile<false, 1, 1, 3>(xb, wb, y, hb, M, Nrows, K, ldc, F, s);
-    if (Nrows < 2048 || ((M + 127) / 128) * ((Nrows + 127) / 128) <= 256)
+    if (t.rows == 64)
       return run_dense_tile<false, 1, 2, 2>(xb, wb, y, hb, M, Nrows, K, ldc, F, s);
   }
   return run_dense_tile<GEGLU, 2, 2, 2>(xb, wb, y, hb, M, Nrows, K, ldc, F, s);

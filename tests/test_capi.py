@@ -294,6 +294,23 @@ def test_gemm_routing():
     assert route(256, big_n, 1024, 2) == -1
 
 
+def test_dense_tiles():
+    """The dense bf16 GEMM takes 64 x 128 tiles above 640 of 64 x 64 only where
+    they leave a CU less than twice as many as 128 x 128 ones."""
+    L = _lib.lib()
+
+    def tile(m, n):
+        t = L.glypr_internal_dense_tile(ctypes.c_int64(m), ctypes.c_int64(n))
+        return t >> 16, t & 0xFFFF
+    assert tile(1, 1) == (64, 64) and tile(2560, 1024) == (64, 64)
+    assert tile(2561, 1024) == (64, 128) and tile(2500, 1280) == (64, 128)
+    for m, n in [(4000, 1280), (8190, 1280), (12000, 768), (8190, 512), (12000, 512)]:
+        assert tile(m, n) == (64, 128), (m, n)
+    for m, n in [(6000, 1280), (12000, 1280), (10000, 768), (16384, 768), (16384, 512),
+                 (8190, 1536), (5000, 2304), (16384, 2048)]:
+        assert tile(m, n) == (128, 128), (m, n)
+
+
 # ---- the model-config struct: C header, ctypes mirror and the Rust binding ----
 
 _C_FIELDS = re.compile(r"^\s*(int64_t|float|double|const uint8_t\*)\s+(\w+);", re.M)
