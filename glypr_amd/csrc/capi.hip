@@ -834,12 +834,19 @@ int glypr_hip_int8_cosine(glypr_hip_ctx* ctx, const int8_t* a, int64_t na, const
   return GLYPR_OK;
 }
 
-// Not part of the public header: the INT8_EXACT GEMM route (GEMM_ROUTE_*) for a
+// Not part of the public header: the int8 GEMM route (GEMM_ROUTE_*) for a
 // shape, and whether the prologue-fused kernel takes it, so host tests can pin
 // the routing without a GPU.
 int glypr_internal_gemm_i8_route(int64_t m, int64_t n, int64_t k, int prologue) {
   if (prologue == 1 || prologue == 2) return gemm_i8_pro_ok(m, n, k, prologue == 2) ? 4 : -1;
   return gemm_i8_route(m, n, k);
+}
+
+// Likewise the kernel and tile (GEMM_TILE_*) that run a plain int8 GEMM, and whether
+// the per-layer-embedding gate runs as one launch.
+int glypr_internal_gemm_i8_tile(int64_t m, int64_t n, int64_t k) { return gemm_i8_tile(m, n, k); }
+int glypr_internal_gemm_i8_gate_ok(int64_t m, int64_t p, int64_t k) {
+  return gemm_i8_gate_ok(m, p, k);
 }
 
 // Likewise the dense bf16 GEMM's tile: rows << 16 | columns.

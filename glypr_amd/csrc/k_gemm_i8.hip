@@ -1326,7 +1326,7 @@ gemm_i8_big_kernel(const int8_t* __restrict__ A, const float* __restrict__ dA,
 }
 
 template <int WMW, int WNW, int TN, bool GEGLU, bool F2>
-hipError_t run_big_tile(const int8_t* xq, const float* dx, const int8_t* wq, const float* dw,
+hipError_t run_big(const int8_t* xq, const float* dx, const int8_t* wq, const float* dw,
                         float* y, int8_t* hq, float* dh, int64_t M, int64_t Nrows, int64_t K,
                         int64_t ldc, int64_t F, hipStream_t s) {
   constexpr int BM = 32 * WMW, BN = 32 * TN * WNW;
@@ -1337,8 +1337,8 @@ hipError_t run_big_tile(const int8_t* xq, const float* dx, const int8_t* wq, con
   return hipGetLastError();
 }
 
-// The plain GEMM's tile: 0 = 128 x 128 (wave 32 x 128), 1 = 64 x 64 (32 x 32),
-// 2 = 64 x 128 (32 x 64).  A wave's column tile and K block (one MFMA and its
+// The large-M plain GEMM's tile: 0 = 128 x 128 (wave 32 x 128), 1 = 64 x 64 (32 x
+// 32), 2 = 64 x 128 (32 x 64).  A wave's column tile and K block (one MFMA and its
 // exact epilogue) costs 0.15-0.2 us alone on its SIMD and ~0.1-0.13 us of a
 // shared one, so what decides is how the grid's waves spread: the estimate below
 // (us, with the measured cost per tile-block for 1 .. 4 workgroups per CU)
@@ -1359,31 +1359,18 @@ inline double big_cost(int64_t M, int64_t N, int64_t K, int tile) {
   return 3.0 + blocks * (rounds * f[fit - 1] + (rest ? f[rest - 1] : 0.0)) +
          (tile == 1 ? 0.0 : (double)(rounds + (rest != 0) - 1));
 }
-inline int big_tile(int64_t M, int64_t N, int64_t K) {
+inline GemmI8Tile big_tile(int64_t M, int64_t N, int64_t K) {
   const double c0 = big_cost(M, N, K, 0), c1 = big_cost(M, N, K, 1), c2 = big_cost(M, N, K, 2);
-  return c1 <= c0 && c1 <= c2 ? 1 : c2 < c0 ? 2 : 0;
+  return c1 <= c0 && c1 <= c2 ? GEMM_TILE_64x64 : c2 < c0 ? GEMM_TILE_64x128 : GEMM_TILE_128x128;
 }
-// Whether up to 2048 rows the 64 x 64 tiles beat gemm_i8_small_kernel, whose
-// 16 x 32 tiles cost 2.7 us + 0.21 us per thousand 32 x 32 x 32 blocks (1213 x
-// 768 x 1280: 9.5 -> 8.3 us; 2048 x 512 x 3072: 22.2 -> 15.5; 1213 x 768 x 768
-// stays: 7.7 against 8.2).
+// Whether up to 2048 rows the large-M kernel takes over from gemm_i8_small_kernel
+// (on the tile big_tile then names), whose 16 x 32 tiles cost 2.7 us + 0.21 us per
+// thousand 32 x 32 x 32 blocks: where 64 x 64 tiles are below that (1213 x 768 x
+// 1280: 9.5 -> 8.3 us in 64 x 64; 2048 x 512 x 3072: 22.2 -> 15.5 in 128 x 128; 1213
+// x 768 x 768 stays: 7.7 against 8.2).
 inline bool tiles_beat_small(int64_t M, int64_t N, int64_t K) {
   const double work = (double)((M + 31) / 32) * ((N + 31) / 32) * (K / QK);
   return big_cost(M, N, K, 1) < 2.7 + 0.00021 * work;
-}
-
-template <bool GEGLU, bool F2>
-hipError_t run_big(const int8_t* xq, const float* dx, const int8_t* wq, const float* dw,
-                   float* y, int8_t* hq, float* dh, int64_t M, int64_t Nrows, int64_t K,
-                   int64_t ldc, int64_t F, hipStream_t s) {
-  if constexpr (!GEGLU) {
-    const int tile = big_tile(M, Nrows, K);
-    if (tile == 1)
-      return run_big_tile<2, 2, 1, false, F2>(xq, dx, wq, dw, y, hq, dh, M, Nrows, K, ldc, F, s);
-    if (tile == 2)
-      return run_big_tile<2, 2, 2, false, F2>(xq, dx, wq, dw, y, hq, dh, M, Nrows, K, ldc, F, s);
-  }
-  return run_big_tile<4, 1, 4, GEGLU, F2>(xq, dx, wq, dw, y, hq, dh, M, Nrows, K, ldc, F, s);
 }
 
 // The large-M kernel addresses operands with 32-bit offsets.
@@ -1885,21 +1872,36 @@ int gemm_i8_route(int64_t M, int64_t Nrows, int64_t K) {
   return ((M + 127) / 128) * ((Nrows + 127) / 128) >= 512 ? GEMM_ROUTE_REG128 : GEMM_ROUTE_REG64;
 }
 
+GemmI8Tile gemm_i8_tile(int64_t M, int64_t N, int64_t K) {
+  switch (gemm_i8_route(M, N, K)) {
+    case GEMM_ROUTE_SMALL:
+      return big_ok(M, N, K) && tiles_beat_small(M, N, K) ? big_tile(M, N, K) : GEMM_TILE_16x32;
+    case GEMM_ROUTE_BIG:
+      return big_tile(M, N, K);
+    case GEMM_ROUTE_REG128:
+      return GEMM_TILE_REG128;
+    default:
+      return GEMM_TILE_REG64;
+  }
+}
+
 namespace {
 
 template <bool F2>
 hipError_t gemm_i8_routed(const int8_t* xq, const float* dx, const int8_t* wq, const float* dw,
                           float* y, int64_t M, int64_t N, int64_t K, int64_t ldc,
                           hipStream_t s) {
-  switch (gemm_i8_route(M, N, K)) {
-    case GEMM_ROUTE_SMALL:
-      if (big_ok(M, N, K) && tiles_beat_small(M, N, K))
-        return run_big<false, F2>(xq, dx, wq, dw, y, nullptr, nullptr, M, N, K, ldc, 0, s);
+  switch (gemm_i8_tile(M, N, K)) {
+    case GEMM_TILE_16x32:
       return run_small<1, 2, 1, false, F2, 3>(xq, dx, wq, dw, y, nullptr, nullptr, M, N, K, ldc,
                                               0, s);
-    case GEMM_ROUTE_BIG:
-      return run_big<false, F2>(xq, dx, wq, dw, y, nullptr, nullptr, M, N, K, ldc, 0, s);
-    case GEMM_ROUTE_REG128:
+    case GEMM_TILE_64x64:
+      return run_big<2, 2, 1, false, F2>(xq, dx, wq, dw, y, nullptr, nullptr, M, N, K, ldc, 0, s);
+    case GEMM_TILE_64x128:
+      return run_big<2, 2, 2, false, F2>(xq, dx, wq, dw, y, nullptr, nullptr, M, N, K, ldc, 0, s);
+    case GEMM_TILE_128x128:
+      return run_big<4, 1, 4, false, F2>(xq, dx, wq, dw, y, nullptr, nullptr, M, N, K, ldc, 0, s);
+    case GEMM_TILE_REG128:
       return run<128, 128, 2, 2, false, F2>(xq, dx, wq, dw, y, nullptr, nullptr, M, N, K, ldc, 0,
                                             s);
     default:
@@ -1938,7 +1940,7 @@ hipError_t geglu_i8_routed(const int8_t* xq, const float* dx, const int8_t* wq, 
       return run_small<2, 2, 2, true, F2, 3>(xq, dx, wq, dw, nullptr, hq, dh, M, 2 * F, K, 0, F,
                                              s);
     case GEMM_ROUTE_BIG:
-      return run_big<true, F2>(xq, dx, wq, dw, nullptr, hq, dh, M, 2 * F, K, 0, F, s);
+      return run_big<4, 1, 4, true, F2>(xq, dx, wq, dw, nullptr, hq, dh, M, 2 * F, K, 0, F, s);
     case GEMM_ROUTE_REG128:
       return run<128, 128, 2, 2, true, F2>(xq, dx, wq, dw, nullptr, hq, dh, M, 2 * F, K, 0, F, s);
     default:
@@ -1963,9 +1965,8 @@ hipError_t launch_gemm_i8(const int8_t* xq, const float* dx, const int8_t* wq, c
 // large tiles hold no 32 columns of a row in 16-row waves).
 bool gemm_i8_gate_ok(int64_t M, int64_t P, int64_t K) {
   const int64_t nb = K / QK;
-  return gemm_i8_route(M, P, K) == GEMM_ROUTE_SMALL && P % QK == 0 &&
-         (nb == 8 || nb == 16 || nb == 24 || nb == 32) &&
-         !(big_ok(M, P, K) && tiles_beat_small(M, P, K));
+  return gemm_i8_tile(M, P, K) == GEMM_TILE_16x32 && P % QK == 0 &&
+         (nb == 8 || nb == 16 || nb == 24 || nb == 32);
 }
 
 hipError_t launch_gemm_i8_gate(const int8_t* xq, const float* dx, const int8_t* wq,

@@ -294,6 +294,35 @@ def test_gemm_routing():
     assert route(256, big_n, 1024, 2) == -1
 
 
+def test_gemm_tiles():
+    """The kernel that runs a plain int8 GEMM (glypr_internal_gemm_i8_tile), on both
+    sides of the sizes at which it changes; the per-layer-embedding gate is fused
+    exactly where that is the small-M kernel."""
+    L = _lib.lib()
+
+    def tile(m, n, k):
+        return L.glypr_internal_gemm_i8_tile(*map(ctypes.c_int64, (m, n, k)))
+
+    def gate(m, p, k):
+        return L.glypr_internal_gemm_i8_gate_ok(*map(ctypes.c_int64, (m, p, k)))
+    T16x32, T64, T64x128, T128, REG128, REG64 = range(6)
+    assert tile(512, 1280, 768) == T16x32 and tile(1000, 768, 768) == T16x32
+    assert tile(1, 33, 2048) == T16x32 and tile(4096, 64, 96) in (REG128, REG64)
+    assert tile(1213, 1280, 768) == T64 and tile(2500, 768, 768) == T64
+    assert tile(3000, 1280, 768) == T64x128
+    assert tile(16384, 2304, 768) == T128
+    big_n = (1 << 31) // 1024
+    assert tile(512, big_n - 1, 1024) != T16x32 and tile(512, big_n, 1024) == REG128
+    assert tile(4096, big_n, 1024) == REG128
+    for n, k in [(1280, 768), (768, 768), (2304, 768), (2048, 512), (512, 2048), (256, 512)]:
+        seen = [tile(m, n, k) != T16x32 for m in range(1, 2049)]
+        assert seen == sorted(seen), (n, k)    # one line, and past it every row count
+        for m in (1, 333, 1000, 2047, 2048):
+            assert gate(m, n, k) == (tile(m, n, k) == T16x32 and k <= 1024), (m, n, k)
+        assert tile(2049, n, k) in (T64, T64x128, T128) and not gate(2049, n, k)
+    assert not gate(100, 48, 512) and not gate(100, 64, 640)
+
+
 def test_dense_tiles():
     """The dense bf16 GEMM takes 64 x 128 tiles above 640 of 64 x 64 only where
     they leave a CU less than twice as many as 128 x 128 ones."""
