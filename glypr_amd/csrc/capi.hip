@@ -844,7 +844,9 @@ int glypr_internal_gemm_i8_route(int64_t m, int64_t n, int64_t k, int prologue) 
 
 // Likewise the kernel and tile (GEMM_TILE_*) that run a plain int8 GEMM, and whether
 // the per-layer-embedding gate runs as one launch.
-int glypr_internal_gemm_i8_tile(int64_t m, int64_t n, int64_t k) { return gemm_i8_tile(m, n, k); }
+int glypr_internal_gemm_i8_tile(int64_t m, int64_t n, int64_t k, int fma2) {
+  return gemm_i8_tile(m, n, k, fma2 != 0);
+}
 int glypr_internal_gemm_i8_gate_ok(int64_t m, int64_t p, int64_t k) {
   return gemm_i8_gate_ok(m, p, k);
 }

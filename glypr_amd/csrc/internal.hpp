@@ -243,12 +243,13 @@ hipError_t launch_attention(const uint16_t* q16, const uint16_t* k16, const uint
 enum { GEMM_ROUTE_SMALL = 0, GEMM_ROUTE_BIG = 1, GEMM_ROUTE_REG128 = 2, GEMM_ROUTE_REG64 = 3 };
 int gemm_i8_route(int64_t M, int64_t Nrows, int64_t K);
 // The kernel and tile that run the plain GEMM: within GEMM_ROUTE_SMALL the small-M
-// kernel (16 x 32) or, where it is faster, a large-M tile.
+// kernel (16 x 32; the same line with and without fma2) or, where it is faster, a
+// large-M tile.
 enum GemmI8Tile {
   GEMM_TILE_16x32 = 0, GEMM_TILE_64x64, GEMM_TILE_64x128, GEMM_TILE_128x128, GEMM_TILE_REG128,
   GEMM_TILE_REG64
 };
-GemmI8Tile gemm_i8_tile(int64_t M, int64_t N, int64_t K);
+GemmI8Tile gemm_i8_tile(int64_t M, int64_t N, int64_t K, bool fma2);
 // y[m,n] = sum_b ((float)S_b * dw[n,b]) * dx[m,b], sequential over b (exact).
 // fma2 (GLYPR_Q8_INT8_FMA): each block's term is added as
 // fma(round(S_b * dw[n,b]), dx[m,b], acc), one rounding fewer per block.

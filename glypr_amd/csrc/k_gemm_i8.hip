@@ -1345,10 +1345,16 @@ hipError_t run_big(const int8_t* xq, const float* dx, const int8_t* wq, const fl
 // deals the workgroups out over 256 CUs in rounds of what fits a CU.
 // Measured, 128 x 128 -> chosen: 2500 x 768 x 768 19.2 -> 10.0 us (64 x 64),
 // 3000 x 768 x 1280 16.8 -> 13.0 (64 x 128), 4800 x 2048 x 512 44 -> 26,
-// 12000 x 768 x 768 39.6 -> 29.5; 6000 x 768 x 1280 stays (22.9 against 25.5), as
-// do 16384 rows of 1280 or 2304 columns (61 against 63).
+// 12000 x 768 x 768 39.6 -> 29.5, 12000 x 1152 x 768 66.2 -> 55.0 (64 x 64); 128 x 128
+// stays at 6000 x 768 x 1280 (22.9 against 25.5), 16384 x 1152 x 768 (69.7 against
+// 70.9 and 75.4) and 16384 rows of 1280 or 2304 columns (61 against 63).
+// Rows of other than whole 32-column lines cost the wider tiles more (12000 x 768 x
+// 1000: 58.5 in 128 x 128, 52.9 in 64 x 128, 49.0 in 64 x 64), and with the two-op
+// epilogue the 64 x 64 tile, which reads the most LDS per product, 4 % more next to
+// the others (8190 x 768 x 768 26.1 in 128 x 128, 26.9 in 64 x 64).
 inline double big_cost(int64_t M, int64_t N, int64_t K, int tile) {
-  static const double f0[] = {0.15, 0.20}, f1[] = {0.216, 0.29, 0.39, 0.53}, f2[] = {0.17, 0.22};
+  static const double f0[] = {0.15, 0.20}, f1[] = {0.203, 0.273, 0.367, 0.498},
+                      f2[] = {0.18, 0.233};
   const int64_t bm = tile == 0 ? 128 : 64, bn = tile == 1 ? 64 : 128;
   const int fit = tile == 1 ? 4 : 2, cols = tile == 0 ? 4 : tile == 1 ? 1 : 2;
   const double* f = tile == 0 ? f0 : tile == 1 ? f1 : f2;
@@ -1356,18 +1362,20 @@ inline double big_cost(int64_t M, int64_t N, int64_t K, int tile) {
   const int64_t rounds = n / fit;
   const int rest = (int)(n % fit);
   const double blocks = (double)(K / QK) * cols;
-  return 3.0 + blocks * (rounds * f[fit - 1] + (rest ? f[rest - 1] : 0.0)) +
-         (tile == 1 ? 0.0 : (double)(rounds + (rest != 0) - 1));
+  const double c = 3.0 + blocks * (rounds * f[fit - 1] + (rest ? f[rest - 1] : 0.0)) +
+                   (tile == 1 ? 0.0 : (double)(rounds + (rest != 0) - 1));
+  return N % 32 == 0 ? c : c * (tile == 0 ? 1.10 : tile == 2 ? 1.05 : 1.0);
 }
-inline GemmI8Tile big_tile(int64_t M, int64_t N, int64_t K) {
-  const double c0 = big_cost(M, N, K, 0), c1 = big_cost(M, N, K, 1), c2 = big_cost(M, N, K, 2);
+inline GemmI8Tile big_tile(int64_t M, int64_t N, int64_t K, bool fma2) {
+  const double c0 = big_cost(M, N, K, 0), c2 = big_cost(M, N, K, 2),
+               c1 = big_cost(M, N, K, 1) * (fma2 ? 1.04 : 1.0);
   return c1 <= c0 && c1 <= c2 ? GEMM_TILE_64x64 : c2 < c0 ? GEMM_TILE_64x128 : GEMM_TILE_128x128;
 }
 // Whether up to 2048 rows the large-M kernel takes over from gemm_i8_small_kernel
 // (on the tile big_tile then names), whose 16 x 32 tiles cost 2.7 us + 0.21 us per
 // thousand 32 x 32 x 32 blocks: where 64 x 64 tiles are below that (1213 x 768 x
-// 1280: 9.5 -> 8.3 us in 64 x 64; 2048 x 512 x 3072: 22.2 -> 15.5 in 128 x 128; 1213
-// x 768 x 768 stays: 7.7 against 8.2).
+// 1280: 9.5 -> 8.3 us; 2048 x 512 x 3072: 26.0 -> 17.8; 2048 x 2048 x 512: 24.0 ->
+// 21.5; 1213 x 768 x 768 stays: 7.7 against 8.2).
 inline bool tiles_beat_small(int64_t M, int64_t N, int64_t K) {
   const double work = (double)((M + 31) / 32) * ((N + 31) / 32) * (K / QK);
   return big_cost(M, N, K, 1) < 2.7 + 0.00021 * work;
@@ -1872,12 +1880,13 @@ int gemm_i8_route(int64_t M, int64_t Nrows, int64_t K) {
   return ((M + 127) / 128) * ((Nrows + 127) / 128) >= 512 ? GEMM_ROUTE_REG128 : GEMM_ROUTE_REG64;
 }
 
-GemmI8Tile gemm_i8_tile(int64_t M, int64_t N, int64_t K) {
+GemmI8Tile gemm_i8_tile(int64_t M, int64_t N, int64_t K, bool fma2) {
   switch (gemm_i8_route(M, N, K)) {
     case GEMM_ROUTE_SMALL:
-      return big_ok(M, N, K) && tiles_beat_small(M, N, K) ? big_tile(M, N, K) : GEMM_TILE_16x32;
+      return big_ok(M, N, K) && tiles_beat_small(M, N, K) ? big_tile(M, N, K, fma2)
+                                                            : GEMM_TILE_16x32;
     case GEMM_ROUTE_BIG:
-      return big_tile(M, N, K);
+      return big_tile(M, N, K, fma2);
     case GEMM_ROUTE_REG128:
       return GEMM_TILE_REG128;
     default:
@@ -1891,7 +1900,7 @@ template <bool F2>
 hipError_t gemm_i8_routed(const int8_t* xq, const float* dx, const int8_t* wq, const float* dw,
                           float* y, int64_t M, int64_t N, int64_t K, int64_t ldc,
                           hipStream_t s) {
-  switch (gemm_i8_tile(M, N, K)) {
+  switch (gemm_i8_tile(M, N, K, F2)) {
     case GEMM_TILE_16x32:
       return run_small<1, 2, 1, false, F2, 3>(xq, dx, wq, dw, y, nullptr, nullptr, M, N, K, ldc,
                                               0, s);
@@ -1965,7 +1974,7 @@ hipError_t launch_gemm_i8(const int8_t* xq, const float* dx, const int8_t* wq, c
 // large tiles hold no 32 columns of a row in 16-row waves).
 bool gemm_i8_gate_ok(int64_t M, int64_t P, int64_t K) {
   const int64_t nb = K / QK;
-  return gemm_i8_tile(M, P, K) == GEMM_TILE_16x32 && P % QK == 0 &&
+  return gemm_i8_tile(M, P, K, false) == GEMM_TILE_16x32 && P % QK == 0 &&
          (nb == 8 || nb == 16 || nb == 24 || nb == 32);
 }
 

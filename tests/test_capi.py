@@ -300,8 +300,8 @@ def test_gemm_tiles():
     exactly where that is the small-M kernel."""
     L = _lib.lib()
 
-    def tile(m, n, k):
-        return L.glypr_internal_gemm_i8_tile(*map(ctypes.c_int64, (m, n, k)))
+    def tile(m, n, k, fma=0):
+        return L.glypr_internal_gemm_i8_tile(*map(ctypes.c_int64, (m, n, k)), ctypes.c_int(fma))
 
     def gate(m, p, k):
         return L.glypr_internal_gemm_i8_gate_ok(*map(ctypes.c_int64, (m, p, k)))
@@ -311,11 +311,19 @@ def test_gemm_tiles():
     assert tile(1213, 1280, 768) == T64 and tile(2500, 768, 768) == T64
     assert tile(3000, 1280, 768) == T64x128
     assert tile(16384, 2304, 768) == T128
+    # two 64 x 128 tiles for each 128 x 128 one, or more of them than fit at once
+    for m, n, k in [(16384, 768, 1152), (16384, 768, 768), (8190, 1536, 1024),
+                    (12000, 1536, 1024)]:
+        assert tile(m, n, k) == T128 and tile(m, n, k, 1) == T128, (m, n, k)
+    assert tile(12000, 512, 2048) == T64 and tile(12000, 512, 2048, 1) == T128
+    assert tile(8190, 768, 768) == T64 and tile(8190, 768, 768, 1) == T128
+    assert tile(12000, 1000, 768) == T64 and tile(12000, 768, 1152) == T64
     big_n = (1 << 31) // 1024
     assert tile(512, big_n - 1, 1024) != T16x32 and tile(512, big_n, 1024) == REG128
     assert tile(4096, big_n, 1024) == REG128
     for n, k in [(1280, 768), (768, 768), (2304, 768), (2048, 512), (512, 2048), (256, 512)]:
         seen = [tile(m, n, k) != T16x32 for m in range(1, 2049)]
+        assert seen == [tile(m, n, k, 1) != T16x32 for m in range(1, 2049)]
         assert seen == sorted(seen), (n, k)    # one line, and past it every row count
         for m in (1, 333, 1000, 2047, 2048):
             assert gate(m, n, k) == (tile(m, n, k) == T16x32 and k <= 1024), (m, n, k)
