@@ -327,6 +327,11 @@ __device__ __forceinline__ int sm_swz(int r) { return (r >> 1) & 7; }
 // (4-way at K = 512) cost less than the wider rows' address arithmetic (gate/up
 // 333 x 512 -> 2 x 2048: 8.8 natural, 9.5 padded), so those keep the natural pitch.
 constexpr int scale_pitch(int nb) { return nb % 32 == 0 ? nb + 4 : nb; }
+// Floats that `chunks` 16-byte chunks take when they arrive in units of 64 lanes (the
+// last unit's spare lanes write too).  Not a float more: LDS is dealt in 1280 B, and
+// at K = 2048 26 such pieces leave room for four workgroups on a CU, 25 for five
+// (1213 x 2048 x 512 18.2 -> 15.0 us).
+constexpr int scale_floats(int chunks) { return (chunks + 63) / 64 * 256; }
 
 // WM x WN waves; wave (wm, wn) owns rows 16 wm.. and TNW 16-row B tiles.
 // GATE: C is not stored; h = geglu(C, U) (U [M][ldu] f32) leaves as Q8_0 with the
@@ -362,7 +367,7 @@ gemm_i8_small_kernel(const int8_t* __restrict__ A, const float* __restrict__ dA,
   static_assert(!GATE || (!GEGLU && TNW == 1 && WN == 2), "gate tile: one Q8_0 block of h");
   constexpr int SLOT = (BM + BN) * BK;
   __shared__ __attribute__((aligned(16))) uint8_t ring[RING * SLOT];
-  __shared__ __attribute__((aligned(16))) float sc[SA + SB + 256];
+  __shared__ __attribute__((aligned(16))) float sc[scale_floats((SA + SB) / 4)];
   __shared__ float amax_x[GEGLU || GATE ? WN * BM : 1];
 
   const int tid = threadIdx.x, lane = tid & 63;
@@ -618,12 +623,14 @@ gemm_i8_geglu8_kernel(const int8_t* __restrict__ A, const float* __restrict__ dA
   constexpr int K = NB * QK, NST = NB / KB;
   constexpr int NW = 4, BM = 16, BN = 64;
   constexpr int UA = BM / 8, UB = BN / 8, UN = UA + UB;   // 2 + 8 DMA units per stage
-  constexpr int PB = scale_pitch(NB), SA = PB * BM, SB = PB * BN;
+  // (K = 1024: with the row scales padded too five would not fit on a CU, and 300
+  // rows of 1024 -> 2 x 2048 -> 1024 take 23.2 instead of 20.6 us)
+  constexpr int PB = scale_pitch(NB), PA = NB == 32 ? NB : PB, SA = PA * BM, SB = PB * BN;
   static_assert(NB % KB == 0 && NB <= SMALL_NB_MAX, "K must be a multiple of 128, <= 2048");
   static_assert(RING >= 2, "ring needs >= 2 slots");
   constexpr int SLOT = (BM + BN) * BK;
   __shared__ __attribute__((aligned(16))) uint8_t ring[RING * SLOT];
-  __shared__ __attribute__((aligned(16))) float sc[SA + SB + 256];
+  __shared__ __attribute__((aligned(16))) float sc[scale_floats((SA + SB) / 4)];
   __shared__ float amax_w[NW][BM];
 
   const int tid = threadIdx.x, lane = tid & 63;
@@ -637,13 +644,14 @@ gemm_i8_geglu8_kernel(const int8_t* __restrict__ A, const float* __restrict__ dA
     return (nl & 8) ? F + c : c;
   };
 
-  constexpr int NQ = NB / 4, PQ = PB / 4;   // 16-byte chunks of a row: filled, in all
+  // 16-byte chunks of a row: filled, in all
+  constexpr int NQ = NB / 4, PAQ = PA / 4, PQ = PB / 4;
   constexpr int SCH = (SA + SB) / 4;
   for (int c0 = wave * 64; c0 < SCH; c0 += NW * 64) {
     const int c = c0 + lane < SCH ? c0 + lane : SCH - 1;
     const float* src;
     if (c < SA / 4) {
-      const int r = c / PQ, q = c - r * PQ < NQ ? c - r * PQ : NQ - 1;
+      const int r = c / PAQ, q = c - r * PAQ < NQ ? c - r * PAQ : NQ - 1;
       const int gm = m0 + r < M ? m0 + r : M - 1;
       src = dA + (int64_t)gm * NB + 4 * q;
     } else {
@@ -685,7 +693,7 @@ gemm_i8_geglu8_kernel(const int8_t* __restrict__ A, const float* __restrict__ dA
     const int brow = wave * 16 + l16;
     offB[kb] = (BM + brow) * BK + ((ch ^ sm_swz(brow)) << 4) + ((lq & 1) << 3);
   }
-  const float* xrow = sc + (4 * lq) * PB;
+  const float* xrow = sc + (4 * lq) * PA;
   const float* wrow = sc + SA + (wave * 16 + l16) * PB;
   const v4i magic = {MAGIC, MAGIC, MAGIC, MAGIC};
   float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -714,7 +722,7 @@ gemm_i8_geglu8_kernel(const int8_t* __restrict__ A, const float* __restrict__ dA
         v4f xq[4];
 #pragma unroll
         for (int rr = 0; rr < 4; rr++)
-          xq[rr] = *reinterpret_cast<const v4f*>(xrow + rr * PB + st * KB);
+          xq[rr] = *reinterpret_cast<const v4f*>(xrow + rr * PA + st * KB);
         const v4f wq = *reinterpret_cast<const v4f*>(wrow + st * KB);
 #pragma unroll
         for (int kb = 0; kb < KB; kb++) {
@@ -842,7 +850,7 @@ gemm_i8_pro_kernel(const float* __restrict__ X, const float* __restrict__ nw, fl
   static_assert(LPR >= 8 && LPR <= 64 && NB % PARTS == 0, "prologue lane layout");
   __shared__ __attribute__((aligned(16))) uint8_t ring[RING * SLOT];
   __shared__ __attribute__((aligned(16))) uint8_t ares[BM * K];
-  __shared__ __attribute__((aligned(16))) float sc[SA + SB + 256];
+  __shared__ __attribute__((aligned(16))) float sc[SA + scale_floats(SB / 4)];
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1435,7 +1443,7 @@ gemm_i8_qkv_kernel(const int8_t* __restrict__ A, const float* __restrict__ dA,
   static_assert(NB % KB == 0 && NB <= SMALL_NB_MAX, "K must be a multiple of 128, <= 2048");
   static_assert(UB % QKV_NW == 0 && UA <= QKV_NW && BM * QKV_SP * 4 <= SLOT, "layout");
   __shared__ __attribute__((aligned(16))) uint8_t ring[QKV_RING * SLOT];
-  __shared__ __attribute__((aligned(16))) float sc[SA + SB + 256];
+  __shared__ __attribute__((aligned(16))) float sc[scale_floats((SA + SB) / 4)];
   __shared__ float sinv[BM];
 
   const int tid = threadIdx.x, lane = tid & 63;
