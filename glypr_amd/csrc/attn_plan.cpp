@@ -50,6 +50,18 @@ double plan_parts(AttnPlan& p, int64_t blocks, int64_t nkb, double start, double
 
 }  // namespace
 
+// The short kernel's grid is nkv Tp / 16 query rows wide and each of its
+// workgroups walks all T keys alone.  On one kv head that wins up to 1024 rows; more
+// heads fill the CUs several times over, and the partitioned kernels win from
+// 1280 rows of all heads (2 x 2 heads: T = 640, 26.5 against 27.1 us; 850, 40.7
+// against 30.3), unless the walks are short: nkv Tp Tp up to 600,000 (4 x 1 heads:
+// T = 321, 18.5 against 21.4; 512, 28.0 against 24.8; 8 x 1: T = 200, 19.3 against
+// 20.8; 321, 32.0 against 26.0).
+bool attn_short(int64_t Tp, int64_t hd, int64_t nq, int64_t nkv, bool segments) {
+  return hd == 256 && !segments && Tp <= 1024 && nq / nkv <= 3 &&
+         (nkv * Tp <= 1280 || nkv * Tp * Tp <= 600000);
+}
+
 // The choices with their measured starts and tile times (us):
 //   16-query blocks, 3 + 1.3 (head_dim 256) and 6.7 + 3.2 (512): few keys;
 //   64-query blocks (256), 13 + 0.52 per q head of the group: where they fill

@@ -857,6 +857,19 @@ int glypr_internal_dense_tile(int64_t m, int64_t n) {
   return t.rows << 16 | t.cols;
 }
 
+// Likewise what one attention launch runs: out = {short kernel, qs, waves, per, kparts}
+// (AttnPlan; rows 0: one sequence of t padded on its own).
+void glypr_internal_attn_plan(int64_t t, int64_t rows, int64_t nq, int64_t nkv, int64_t hd,
+                              int64_t window, int segments, int* out) {
+  const int64_t tp = rows > 0 ? rows : attn_padded_len(t);
+  const AttnPlan p = attn_plan(t, tp, hd, nq, nkv, window, segments != 0);
+  out[0] = attn_short(tp, hd, nq, nkv, segments != 0);
+  out[1] = p.qs;
+  out[2] = p.waves;
+  out[3] = p.per;
+  out[4] = p.kparts;
+}
+
 static const char* const kKernelNames[GLYPR_K_COUNT] = {
     "quantize",   "rmsnorm_quant",  "gemm_i8", "gemm_i8_geglu", "to_bf16", "rmsnorm_bf16",
     "gemm_bf16",  "gemm_bf16_geglu", "rmsnorm", "geglu",         "gather",  "dequant",

@@ -189,6 +189,8 @@ constexpr int64_t ATTN_MAX_PARTS = 64;
 struct AttnPlan {
   int waves, qs, per, kparts;
 };
+// Whether one sequence runs the single-launch slice kernel instead (k_attn.hip)
+bool attn_short(int64_t Tp, int64_t hd, int64_t nq, int64_t nkv, bool segments);
 AttnPlan attn_plan(int64_t Tseg, int64_t rows, int64_t hd, int64_t nq, int64_t nkv,
                    int64_t window, bool segments);
 inline int64_t attn_padded_len(int64_t t) { return (t + ATTN_TP_ALIGN - 1) / ATTN_TP_ALIGN * ATTN_TP_ALIGN; }

@@ -687,7 +687,6 @@ __global__ void __launch_bounds__(256) attn_combine_kernel(
 constexpr int ASH_WAVES = 8;
 constexpr int ASH_KS = 16;                  // keys per step
 constexpr int ASH_DS = 32;                  // head dims per slice (one Q8_0 block)
-constexpr int64_t ATTN_SHORT_TP = 1024;     // padded lengths it runs up to
 constexpr int ASH_KU = 8;                   // 1 KB K units per step (2 key rows each)
 constexpr int ASH_SLOT_K = ASH_KS * 256 * 2;
 
@@ -981,9 +980,7 @@ static hipError_t run_attention(const f16* q, const f16* k, const f16* v, float*
                                 int64_t nq, int64_t nkv, int64_t window, hipStream_t s,
                                 uint16_t* cb, const int2* seg, int64_t seg_max) {
   const int64_t G = nq / nkv;
-  // (two kv heads double its grid: past 1280 rows of both it takes three rounds
-  // and more, where the tiles win: T = 850, 37.7 against 30.3 us)
-  if (HD == 256 && !seg && Tp <= ATTN_SHORT_TP && nkv * Tp <= 1280 && G <= 3) {
+  if (HD == 256 && attn_short(Tp, HD, nq, nkv, seg != nullptr)) {
     // one short sequence: the single-launch slice kernel
     const int64_t items = nkv * (Tp / 16) * (HD / ASH_DS);
     const unsigned grid = (unsigned)((items + 7) / 8 * 8);
