@@ -22,17 +22,16 @@ int64_t key_tiles(int64_t Tseg, int64_t window, int64_t queries) {
 // workgroups per partition and returns its cost in microseconds: every round
 // of 256 workgroups (one per CU: the K/V ring or the accumulators leave room
 // for one) takes `start` (launch, Q, first tile, epilogue) plus `tile` per key
-// tile, and a split pays for the f32 partials (written, then read by the
-// combine, ~5.5 TB/s) and the combine launch.  A grid that fills a round by
-// itself is never split.
-// `tile_full` takes the place of `tile` past 60 % of the CUs (clocks under load).
+// tile (`tile_full` past 60 % of the CUs: shared L2 reads, clocks), and a split
+// pays for the combine launch and the f32 partials, written and read by the
+// combine at ~8 TB/s.  A grid that fills a round by itself is never split.
 double plan_parts(AttnPlan& p, int64_t blocks, int64_t nkb, double start, double tile,
                   double tile_full, int64_t part_bytes) {
   double best = 0;
   int64_t most = nkb < ATTN_MAX_PARTS ? nkb : ATTN_MAX_PARTS;
   if (blocks >= ATTN_BLOCKS) most = 1;
   for (int64_t want = 1; want <= most; want++) {
-    const double split = want > 1 ? 3.0 + want * part_bytes * 2 / 5.5e6 : 0.0;
+    const double split = want > 1 ? 1.4 + want * part_bytes * 0.24e-6 : 0.0;
     if (want > 1 && start + split >= best) break;   // so do all that follow
     const int64_t per = (nkb + want - 1) / want;
     if ((nkb + per - 1) / per != want) continue;
@@ -62,15 +61,18 @@ bool attn_short(int64_t Tp, int64_t hd, int64_t nq, int64_t nkv, bool segments) 
          (nkv * Tp <= 1280 || nkv * Tp * Tp <= 600000);
 }
 
-// The choices with their measured starts and tile times (us):
-//   16-query blocks, 3 + 1.3 (head_dim 256) and 6.7 + 3.2 (512): few keys;
-//   64-query blocks (256), 13 + 0.52 per q head of the group: where they fill
-//     just one round and the 32 x 32 tiles leave SIMDs idle (32 sequences x 512
-//     rows of 3 heads: 41.7 against 55 us; T = 8192 of 3 heads: 249 against
-//     271 us);
-//   32 x 32 tiles, 5 + 0.8 (0.97 under load) and 11.5 + 2.05: everything longer (T = 1777,
-//     window 512: 49.9 -> 37.0 us with the prologue; T = 4000 of 3 heads: 118 ->
-//     87; T = 4000 of 4 heads, head_dim 512: 375 -> 185; T = 8192: 1472 -> 565).
+// The choices with their starts and tile times (us), fitted to every choice and
+// partition count measured at 301 shapes (64 to 8192 keys, 1 to 8 kv heads of 1 to 4
+// q heads, single sequences and batches); the chosen ones are 0.6 % slower than the
+// best on average:
+//   16-query blocks: few keys;
+//   64-query blocks (head_dim 256): on few q heads, and where they fill just one
+//     round and the 32 x 32 tiles leave SIMDs idle (32 sequences x 512 rows of 3
+//     heads: 39.9 against 55.2 us; T = 8192 of 3 heads: 248 against 268 us; 64
+//     sequences x 128 rows of 2 x 2 heads: 16.3 against 18.0);
+//   32 x 32 tiles: everything longer (T = 1777, window 512: 49.9 -> 37.2 us with the
+//     prologue; T = 3500 of 3 heads: 82 -> 69; T = 4000 of 4 heads, head_dim 512: 375
+//     -> 185; T = 8192: 1472 -> 570).
 AttnPlan attn_plan(int64_t Tseg, int64_t rows, int64_t hd, int64_t nq, int64_t nkv,
                    int64_t window, bool segments) {
   const int64_t G = nq / nkv, part_bytes = rows * nq * hd * 4;
@@ -87,16 +89,19 @@ AttnPlan attn_plan(int64_t Tseg, int64_t rows, int64_t hd, int64_t nq, int64_t n
     }
   };
   const bool wide = hd == 512;
-  offer(0, 1, 16, rows / 16, wide ? 6.7 : 3.0, wide ? 3.2 : 1.3,
-        wide ? 3.2 : 1.3);
-  if (!wide) offer(0, 4, 64, rows / 64, 13.0, 0.52 * G, 0.52 * G);
+  if (wide) {
+    offer(0, 1, 16, rows / 16, 4.3, 2.14, 2.14);
+  } else {
+    offer(0, 1, 16, rows / 16, 6.9, 0.73, 0.88);
+    offer(0, 4, 64, rows / 64, 7.2, 0.72 * G, 0.51 * G > 0.92 ? 0.51 * G : 0.92);
+  }
   // Four column groups (32 queries of one head) per workgroup fill its CU's
   // SIMDs.  With several sequences a workgroup stays within one, so within 64
   // rows: two groups of one head, three of three heads.
   const int waves = !segments || G % 2 == 0 ? 4 : G == 1 ? 2 : 3;
   const int64_t queries = waves % G == 0 ? 32 * (waves / G) : 64;
-  offer(waves, 0, queries, ((rows >> 5) * G + waves - 1) / waves, wide ? 11.5 : 5.0,
-        wide ? 2.05 : 0.8, wide ? 2.05 : 0.97);
+  offer(waves, 0, queries, ((rows >> 5) * G + waves - 1) / waves, wide ? 6.3 : 8.3,
+        wide ? 1.94 : 0.91, wide ? 1.74 : 0.88);
   return best;
 }
 
