@@ -39,24 +39,17 @@ __device__ __forceinline__ int key_of_row(int r) {
   return (r & 19) | ((r & 4) << 1) | ((r & 8) >> 1);
 }
 
-// O^T accumulators.  HD 512 keeps its 256 accumulator registers per lane in
-// AGPRs (the other 256 registers hold Q and the tile in work), which only an
-// asm operand pins; s_nop 1 covers a vector ALU write of an operand right in
+// O^T accumulators stay in AGPRs (HD 512: all 256 of a lane, while the other 256
+// registers hold Q and the tile in work), which only an asm operand pins; s_nop 1 covers a vector ALU write of an operand right in
 // front, and acc_settle the reads of o behind the last product.
-template <int HD>
 __device__ __forceinline__ void pv_mfma(v16f& o, const v8h& a, const v8h& b) {
-  if constexpr (HD >= 256)
-    asm("s_nop 1\n\tv_mfma_f32_32x32x16_f16 %0, %1, %2, %0" : "+a"(o) : "v"(a), "v"(b));
-  else
-    o = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, o, 0, 0, 0);
+  asm("s_nop 1\n\tv_mfma_f32_32x32x16_f16 %0, %1, %2, %0" : "+a"(o) : "v"(a), "v"(b));
 }
-template <int HD, int NT>
+template <int NT>
 __device__ __forceinline__ void acc_settle(v16f (&o)[NT]) {
-  if constexpr (HD >= 256) {
-    asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
+  asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
 #pragma unroll
-    for (int t = 0; t < NT; t++) asm volatile("" : "+a"(o[t]));
-  }
+  for (int t = 0; t < NT; t++) asm volatile("" : "+a"(o[t]));
 }
 
 template <int HD, int NWV, bool DIRECT>
@@ -217,12 +210,12 @@ attn_tile32_kernel(const f16* __restrict__ q16, const f16* __restrict__ kk,
         const float alpha = __expf(m_run - m_use);
         l_run *= alpha;
         l_lo *= alpha;
-        acc_settle<HD>(o);
+        acc_settle(o);
 #pragma unroll
         for (int t = 0; t < NT; t++) {
 #pragma unroll
           for (int r = 0; r < 16; r++) o[t][r] *= alpha;
-          if constexpr (HD >= 256) asm volatile("" : "+a"(o[t]));
+          asm volatile("" : "+a"(o[t]));
         }
       }
       m_run = m_new;
@@ -248,7 +241,7 @@ attn_tile32_kernel(const f16* __restrict__ q16, const f16* __restrict__ kk,
     };
     // S^T of tile kb+1 (past the last tile: stale LDS, unused) over the
     // exponentials of tile kb, then O^T += V^T P^T; fragments one chunk ahead
-    constexpr int CH = HD == 512 ? 4 : 4;
+    constexpr int CH = 4;
     v8h fr[2][CH];
     float ps[2] = {0.0f, 0.0f};
 #pragma unroll
@@ -288,7 +281,7 @@ attn_tile32_kernel(const f16* __restrict__ q16, const f16* __restrict__ kk,
 #pragma unroll
       for (int e = 0; e < CH; e++) {
         const int i = c * CH + e;
-        pv_mfma<HD>(o[i >> 1], fr[(c + PB) & 1][e], pf[i & 1]);
+        pv_mfma(o[i >> 1], fr[(c + PB) & 1][e], pf[i & 1]);
       }
       __builtin_amdgcn_sched_barrier(0);
     }
@@ -296,7 +289,7 @@ attn_tile32_kernel(const f16* __restrict__ q16, const f16* __restrict__ kk,
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   l_run = pair_sum32(l_run + l_lo);
-  acc_settle<HD>(o);
+  acc_settle(o);
 
   if (c0 + w >= c1) return;   // a spare wave (no barrier follows)
   // O^T tile t, register r: dim 32 t + 8 (r >> 2) + 4 lh + (r & 3) of query qi
@@ -307,7 +300,7 @@ attn_tile32_kernel(const f16* __restrict__ q16, const f16* __restrict__ kk,
     const int64_t rowoff = (int64_t)qi * width + (int64_t)h * HD;
 #pragma unroll
     for (int t = 0; t < NT; t++) {
-      if constexpr (HD >= 256) asm volatile("" : "+a"(o[t]));
+      asm volatile("" : "+a"(o[t]));
       float y[16];
 #pragma unroll
       for (int r = 0; r < 16; r++) y[r] = o[t][r] * inv;
@@ -348,7 +341,7 @@ attn_tile32_kernel(const f16* __restrict__ q16, const f16* __restrict__ kk,
   float* po = part_o + prow * nq * HD + (int64_t)h * HD;
 #pragma unroll
   for (int t = 0; t < NT; t++) {
-    if constexpr (HD >= 256) asm volatile("" : "+a"(o[t]));
+    asm volatile("" : "+a"(o[t]));
 #pragma unroll
     for (int c = 0; c < 4; c++)
       *reinterpret_cast<v4f*>(po + 32 * t + 8 * c + 4 * lh) =

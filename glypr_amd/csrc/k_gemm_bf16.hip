@@ -506,7 +506,7 @@ inline bool big_ok(int64_t M, int64_t Nrows, int64_t K) {
 // geglu(gate, up) leaves as bf16.
 // ---------------------------------------------------------------------------
 template <bool GEGLU, int TM, int TN, int BKE, int RING, bool VEC>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RING * (TM + TN) > 10 ? 1 : 2)))
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
 gemm_bf16w_kernel(const uint16_t* __restrict__ A, const uint16_t* __restrict__ B,
                   float* __restrict__ C, uint16_t* __restrict__ Hb, int M, int N, int K,
                   int ldc, int F, int tiles_n) {

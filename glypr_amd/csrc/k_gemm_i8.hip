@@ -1261,8 +1261,8 @@ gemm_i8_big_kernel(const int8_t* __restrict__ A, const float* __restrict__ dA,
     // lane derives and stores.  The int8 rows leave as dwords: a 4 x 4 byte
     // transpose inside each quad of lanes turns four rows' bytes of one column
     // into four columns of one row.
-    constexpr int NP = TN / 2, TE = 32 * NP;   // table entries
-    static_assert(TN % 2 == 0 && TE <= 64, "gate and up tiles in pairs, one entry per lane");
+    constexpr int NP = 2, TE = 64;   // h blocks of a wave; table entries, one per lane
+    static_assert(TN == 2 * NP, "gate and up tiles in pairs");
     const int nbh = F / QK;
     uint32_t* tab =
         reinterpret_cast<uint32_t*>(ring + (((nst - 1) & 1) ^ 1) * SLOT) + wave * TE * 2;
@@ -1294,11 +1294,11 @@ gemm_i8_big_kernel(const int8_t* __restrict__ A, const float* __restrict__ dA,
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     const int c = hc0 + wn * 16 * TN;
-    if (TE >= 64 || lane < TE) {
+    {
       const QScale q = q8_scale(__uint_as_float(tab[lane]));
       tab[TE + lane] = __float_as_uint(q.id);
-      const int e_half = lane / (16 * NP), e_p = (lane >> 3) & (NP - 1);
-      const int r = 2 * (lane & 7) + ((lane / (8 * NP)) & 1);
+      const int e_half = lane >> 5, e_p = (lane >> 3) & 1;
+      const int r = 2 * (lane & 7) + ((lane >> 4) & 1);
       const int gm = m0 + wm * 32 + 4 * e_half + 8 * (r >> 2) + (r & 3), hb = c + 32 * e_p;
       if (gm < M && hb < F) dH[(int64_t)gm * nbh + (hb >> 5)] = q.dq;
     }
