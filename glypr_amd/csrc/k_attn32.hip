@@ -11,15 +11,16 @@
 // issue over the exponentials of tile kb, fragments four MFMAs ahead of use;
 // one barrier per tile.
 //
-// What bounds it: LDS.  Every MFMA reads one 1 KB fragment, and a CU's LDS
-// serves 150 B/ns (64 B/clock, measured with conflict-free ds_read_b128 from
-// four or eight waves): per tile and CU 256 KB (HD 512) take 1.75 us of the
-// ~2.0 us, the 64 MFMAs per wave 1.1 us.  T = 8192, 4 heads on one kv head of
-// 512: 1350 + 59 us (16-query blocks, 4 partitions, combine) -> 510 us in one
-// launch, 1.08 PFLOP/s of the card's 1.36 for a large f16 product; the whole
-// call 1472 -> 565 us.  T = 1777, window 512, 2 x 2 heads of 256: 49.9 -> 37.0 us
-// (the tile loop is 11 us of it, Q and first tile 5, partials 4, the prologue
-// and combine launches 16).
+// What bounds it: the one wave of each SIMD.  At T = 8192, 4 heads on one kv head
+// of 512, the MFMAs take 47 % of the SIMD cycles (64 of 32 clocks per tile and wave,
+// at the 1.8 GHz the card holds under them), 23 % of the wave's time are waits at the
+// tile's barrier and for fragments, 13 % VALU, and nothing else runs on the
+// SIMD meanwhile.  LDS is not it: the fragment reads are 23 % of its cycles (a
+// conflict-free ds_read_b128 takes 4 clocks, 256 B/clock per CU) without one bank
+// conflict.  Same shape: 1350 + 59 us (16-query blocks, 4 partitions, combine) ->
+// 553 us in one launch, 0.99 PFLOP/s of the card's 1.36 for a large f16 product; the
+// whole call 1472 -> 594 us.  T = 1777, window 512, 2 x 2 heads of 256: 49.9 -> 37.3 us
+// (the tile kernel 22.8, the prologue and combine launches 8.3 and 7.1).
 #include "attn_common.hpp"
 #include "device_common.hpp"
 #include "internal.hpp"
@@ -117,7 +118,8 @@ attn_tile32_kernel(const f16* __restrict__ q16, const f16* __restrict__ kk,
   // c ^ (key_of_row(r) & 15)); V^T unit u = dim rows 16 u .. 16 u + 15 (chunk
   // c of row r at c ^ ((r >> 2) & 3)).  LDS serves a ds_read_b128 in groups of
   // 16 lanes (0-3, 12-15, 20-27 and the other 16, then the upper half alike)
-  // over 64 banks: both swizzles give a group's rows distinct banks.
+  // over 64 banks: both swizzles give a group's rows distinct banks (for these 32-row
+  // fragments; (r >> 1) & 3, right for the 16-row ones, halves the V^T rate).
   const int krow = lane / KLPR;
   const int kl = krow * HD * 2 + (((lane % KLPR) ^ krow) << 4);
   const int vl = (lane >> 2) * Tp * 2 + (((lane & 3) ^ ((lane >> 4) & 3)) << 4);

@@ -1976,8 +1976,9 @@ hipError_t launch_gemm_i8(const int8_t* xq, const float* dx, const int8_t* wq, c
 }
 
 // The PLE gate with its GeGLU and Q8_0 epilogue: where the plain product would
-// take gemm_i8_small_kernel, at the widths it is built for, with h in whole
-// Q8_0 blocks.  333 x 512 x 256: 6.3 us of two launches -> 4.8, and a layer's
+// take gemm_i8_small_kernel, at the widths it is built for (hidden 256 to 1024 by
+// 256: an instance each; others keep the two launches), with h in whole Q8_0
+// blocks.  333 x 512 x 256: 6.3 us of two launches -> 4.8, and a layer's
 // chain has one dependent launch less.  More rows keep the two launches (the product's
 // large tiles hold no 32 columns of a row in 16-row waves).
 bool gemm_i8_gate_ok(int64_t M, int64_t P, int64_t K) {

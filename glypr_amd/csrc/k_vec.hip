@@ -370,7 +370,9 @@ hipError_t run_int8_pairs_mt(const int8_t* a, int64_t na, const int8_t* b, int64
 constexpr int64_t PAIRS_WG = 512;
 
 // The LDS kernel for rows of 64, 128, 256, 512, 768 or 1024 bytes (the MRL
-// dims); up to 8 workgroups per CU, each walking the tiles that are left.
+// dims: every width is an instance of its own per query count and product, so
+// others keep int8_pairs_kernel); the workgroups that fit at once, each walking
+// the tiles that are left.
 template <int MT, bool COS>
 bool run_int8_pairs_lds(const int8_t* a, int64_t na, const int8_t* b, int64_t nb, int64_t dim,
                         int32_t* out_d, float* out_c, hipStream_t s) {
