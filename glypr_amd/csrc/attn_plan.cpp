@@ -21,17 +21,21 @@ int64_t key_tiles(int64_t Tseg, int64_t window, int64_t queries) {
 // Sets the cheapest of 1 .. most partitions over nkb key tiles for `blocks`
 // workgroups per partition and returns its cost in microseconds: every round
 // of 256 workgroups (one per CU: the K/V ring or the accumulators leave room
-// for one) takes `start` (launch, Q, first tile, epilogue) plus `tile` per key
-// tile (`tile_full` past 60 % of the CUs: shared L2 reads, clocks), and a split
-// pays for the combine launch and the f32 partials, written and read by the
-// combine at ~8 TB/s.  A grid that fills a round by itself is never split.
+// for one; two of two waves at head_dim 256 fit and count as one) takes `start`
+// (launch, Q, first tile, epilogue) plus `tile` per key tile (`tile_full` past 60 %
+// of the CUs: shared L2 reads, clocks), and a split pays for the combine launch and
+// the f32 partials, written and read by the combine at ~8.7 TB/s (past 34 MB, which
+// the caches do not hold, at 5.7).  A grid that fills a round by itself is never
+// split.
 double plan_parts(AttnPlan& p, int64_t blocks, int64_t nkb, double start, double tile,
                   double tile_full, int64_t part_bytes) {
+  const double mb = part_bytes * 1e-6;
   double best = 0;
   int64_t most = nkb < ATTN_MAX_PARTS ? nkb : ATTN_MAX_PARTS;
   if (blocks >= ATTN_BLOCKS) most = 1;
   for (int64_t want = 1; want <= most; want++) {
-    const double split = want > 1 ? 1.4 + want * part_bytes * 0.24e-6 : 0.0;
+    const double out = want * mb;
+    const double split = want > 1 ? 1.2 + out * 0.23 + (out > 34 ? (out - 34) * 0.12 : 0.0) : 0.0;
     if (want > 1 && start + split >= best) break;   // so do all that follow
     const int64_t per = (nkb + want - 1) / want;
     if ((nkb + per - 1) / per != want) continue;
@@ -62,8 +66,8 @@ bool attn_short(int64_t Tp, int64_t hd, int64_t nq, int64_t nkv, bool segments) 
 }
 
 // The choices with their starts and tile times (us), fitted to every choice and
-// partition count measured at 301 shapes (64 to 8192 keys, 1 to 8 kv heads of 1 to 4
-// q heads, single sequences and batches); the chosen ones are 0.6 % slower than the
+// partition count measured at 587 shapes (64 to 8192 keys, 1 to 8 kv heads of 1 to 4
+// q heads, single sequences and batches); the chosen ones are 0.4 % slower than the
 // best on average:
 //   16-query blocks: few keys;
 //   64-query blocks (head_dim 256): on few q heads, and where they fill just one
@@ -72,17 +76,18 @@ bool attn_short(int64_t Tp, int64_t hd, int64_t nq, int64_t nkv, bool segments) 
 //     sequences x 128 rows of 2 x 2 heads: 16.3 against 18.0);
 //   32 x 32 tiles: everything longer (T = 1777, window 512: 49.9 -> 37.2 us with the
 //     prologue; T = 3500 of 3 heads: 82 -> 69; T = 4000 of 4 heads, head_dim 512: 375
-//     -> 185; T = 8192: 1472 -> 594).
+//     -> 185; T = 8192: 1460 -> 573).
 AttnPlan attn_plan(int64_t Tseg, int64_t rows, int64_t hd, int64_t nq, int64_t nkv,
                    int64_t window, bool segments) {
   const int64_t G = nq / nkv, part_bytes = rows * nq * hd * 4;
   AttnPlan best{};
   double best_cost = 0;
   auto offer = [&](int waves, int qs, int64_t queries, int64_t blocks, double start,
-                   double tile, double tile_full) {
+                   double tile, double tile_full, int fit = 1) {
     AttnPlan p{waves, qs, 0, 0};
-    const double c = plan_parts(p, nkv * blocks, key_tiles(Tseg, window, queries), start, tile,
-                                tile_full, part_bytes);
+    const double c = plan_parts(p, (nkv * blocks + fit - 1) / fit,
+                                key_tiles(Tseg, window, queries), start, tile, tile_full,
+                                part_bytes);
     if (best.kparts == 0 || c < best_cost) {
       best = p;
       best_cost = c;
@@ -90,18 +95,19 @@ AttnPlan attn_plan(int64_t Tseg, int64_t rows, int64_t hd, int64_t nq, int64_t n
   };
   const bool wide = hd == 512;
   if (wide) {
-    offer(0, 1, 16, rows / 16, 4.3, 2.14, 2.14);
+    offer(0, 1, 16, rows / 16, 2.1, 2.25, 2.25);
   } else {
-    offer(0, 1, 16, rows / 16, 6.9, 0.73, 0.88);
-    offer(0, 4, 64, rows / 64, 7.2, 0.72 * G, 0.51 * G > 0.92 ? 0.51 * G : 0.92);
+    offer(0, 1, 16, rows / 16, 6.3, 0.84, 0.89);
+    // (16 waves share the tiles at 4 heads: far slower once the CUs are full)
+    offer(0, 4, 64, rows / 64, 6.6, 0.85 * G, G < 4 ? 1.0 : 5.0);
   }
   // Four column groups (32 queries of one head) per workgroup fill its CU's
   // SIMDs.  With several sequences a workgroup stays within one, so within 64
   // rows: two groups of one head, three of three heads.
   const int waves = !segments || G % 2 == 0 ? 4 : G == 1 ? 2 : 3;
   const int64_t queries = waves % G == 0 ? 32 * (waves / G) : 64;
-  offer(waves, 0, queries, ((rows >> 5) * G + waves - 1) / waves, wide ? 6.3 : 8.3,
-        wide ? 1.94 : 0.91, wide ? 1.74 : 0.88);
+  offer(waves, 0, queries, ((rows >> 5) * G + waves - 1) / waves, wide ? 4.8 : 8.8,
+        wide ? 2.0 : 0.77, wide ? 1.72 : 0.68, waves == 2 && !wide ? 2 : 1);
   return best;
 }
 

@@ -25,7 +25,9 @@ def test_partitioned_choices():
             (128, 4, 2, 256, 512, 8192, "q64"), (64, 1, 1, 256, 0, 6400, "q64"),
             (64, 4, 2, 256, 512, 6400, "q64"), (200, 3, 1, 256, 0, 3072, "q16"),
             (512, 3, 1, 256, 0, 16384, "q64"), (426, 3, 1, 256, 0, 5440, "tile"),
-            (512, 4, 1, 512, 0, 16384, "tile")]:
+            (512, 4, 1, 512, 0, 16384, "tile"), (1500, 4, 1, 512, 0, 4608, "tile"),
+            (512, 4, 1, 256, 0, 16384, "tile"), (400, 4, 4, 256, 0, 4480, "tile"),
+            (128, 4, 4, 256, 0, 8192, "tile")]:
         p = plan(t, nq, nkv, hd, w, rows=rows, segments=True)
         assert (p.kind, p.kparts) == (kind, 1), (t, nq, nkv, hd, rows, p)
     for t, nq, nkv, hd, w, kind, kparts in [

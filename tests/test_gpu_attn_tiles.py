@@ -88,10 +88,10 @@ def test_tile_attention_batch_vs_single(ctx, oracle, nq, nkv, lens):
     # bands of at most a wave's 32 queries, with partial tiles and column groups
     (4161, 31, 3, 1, 256, False), (4225, 1, 2, 1, 256, False), (2113, 33, 8, 2, 256, False),
     (4225, 31, 4, 4, 256, False), (4161, 33, 2, 1, 512, False), (4225, 31, 3, 1, 512, False),
-    (2113, 1, 8, 2, 512, False), (1105, 31, 4, 4, 512, False), (2113, 64, 2, 2, 512, True),
+    (2113, 1, 8, 2, 512, False), (1301, 31, 4, 4, 512, False), (2113, 64, 2, 2, 512, True),
     # one to four q heads per kv head, one partition and several
     (2081, 0, 1, 1, 256, True), (2113, 0, 2, 1, 256, True), (1089, 512, 3, 1, 256, True),
-    (1153, 0, 4, 1, 256, True), (2690, 512, 6, 2, 256, False), (2113, 512, 8, 2, 256, False),
+    (1153, 0, 4, 1, 256, True), (3500, 512, 6, 2, 256, False), (2113, 512, 8, 2, 256, False),
     (577, 0, 1, 1, 512, True), (643, 0, 2, 1, 512, True), (671, 0, 3, 1, 512, True),
     (705, 512, 8, 2, 512, True), (2689, 512, 6, 2, 512, False)])
 def test_planned_tiles_vs_oracle(ctx, oracle, t, window, nq, nkv, hd, split):
@@ -104,17 +104,18 @@ def test_planned_tiles_vs_oracle(ctx, oracle, t, window, nq, nkv, hd, split):
 
 @pytest.mark.parametrize("nq,nkv,hd,window,lens,waves,split", [
     (1, 1, 256, 0, [2000, 1900, 64, 1, 1700, 31], 2, True),
-    (2, 2, 256, 0, [1500, 2, 63, 1700, 65, 1024, 333], 2, False),
+    (2, 2, 256, 0, [1500, 2, 63, 1700, 65, 1024, 333], 2, True),
+    (2, 2, 256, 200, [1000, 65, 999, 64, 1000, 960, 1, 900, 1000, 800, 31, 930], 2, False),
     (2, 1, 256, 200, [1500, 2, 63, 1700, 65, 1024, 333], 4, True),
-    (3, 1, 256, 0, [1000, 64, 31, 700, 900, 1, 130], 3, True),
+    (3, 1, 256, 0, [2000, 64, 1, 333], 3, True),
     (3, 1, 256, 200, [1500, 2, 63, 1700, 65, 1024, 333], 3, False),
     (4, 1, 256, 200, [2000, 1900, 64, 1, 1700, 31], 4, False),
     (1, 1, 512, 0, [400, 5, 128, 300, 33, 1, 500, 257], 2, True),
     (2, 2, 512, 0, [2000, 1900, 64, 1, 1700, 31], 2, False),
     (2, 1, 512, 0, [1000, 64, 31, 700, 900, 1, 130], 4, True),
-    (3, 1, 512, 0, [1500, 2, 63, 1700, 65, 1024, 333], 3, True),
+    (3, 1, 512, 0, [1000, 64, 31, 700, 900, 1, 130], 3, True),
     (6, 2, 512, 0, [1000, 64, 31, 700, 900, 1, 130], 3, False),
-    (4, 1, 512, 0, [400, 5, 128, 300, 33, 1, 500, 257], 4, True),
+    (4, 1, 512, 0, [600, 64, 1, 550, 33, 500, 31], 4, True),
     (4, 2, 512, 0, [1500, 2, 63, 1700, 65, 1024, 333], 4, False)])
 def test_planned_tiles_batch_vs_single(ctx, oracle, nq, nkv, hd, window, lens, waves, split):
     """One attention layer with its feed-forward block silenced (ffn_down = 0), so
