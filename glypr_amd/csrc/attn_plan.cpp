@@ -76,7 +76,7 @@ bool attn_short(int64_t Tp, int64_t hd, int64_t nq, int64_t nkv, bool segments) 
 //     sequences x 128 rows of 2 x 2 heads: 16.3 against 18.0);
 //   32 x 32 tiles: everything longer (T = 1777, window 512: 49.9 -> 37.2 us with the
 //     prologue; T = 3500 of 3 heads: 82 -> 69; T = 4000 of 4 heads, head_dim 512: 375
-//     -> 185; T = 8192: 1460 -> 573).
+//     -> 185; T = 8192: 1472 -> 594).
 AttnPlan attn_plan(int64_t Tseg, int64_t rows, int64_t hd, int64_t nq, int64_t nkv,
                    int64_t window, bool segments) {
   const int64_t G = nq / nkv, part_bytes = rows * nq * hd * 4;
